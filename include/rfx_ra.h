@@ -83,7 +83,7 @@ uint64_t rfx_ctx_workspace_bytes(rfx_ctx* ctx);
  * (keys per thread of the onesweep tile: 8, 12 or 16, for 4/8-byte keys
  * with 0/4/8-byte values), "sort.digit" (radix digit bits, 8, 9 or 10, for
  * the same shapes; 0 chooses from key_bits: 9 for 17-18 bits, 10 for
- * 19-20, else 8), "join.fb_tile" and "join.ex_tile" (2048 or 4096 merged
+ * 19-20, 6 for 21-24, 7 for 25-28, else 8), "join.fb_tile" and "join.ex_tile" (2048 or 4096 merged
  * items per find_bounds / expansion tile), "select.vt" (rows per thread of
  * the select pass: 8, 16, 24 or 32), "mapfilter.mode" (1: run programs
  * compiled for their types only, 2: interpret them only; the default 0

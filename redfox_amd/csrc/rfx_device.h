@@ -181,6 +181,18 @@ __device__ __forceinline__ T wave_incl_scan(T x) {
   }
   return x;
 }
+// The same sum of 32-bit words by DPP (row shifts, then row broadcasts):
+// six adds instead of six LDS permutes.  Every lane must be active.
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  int x = static_cast<int>(v);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return static_cast<uint32_t>(x);
+}
 // This thread's wave within its block.  The same for every lane, and said
 // so with readfirstlane: values derived from it (wave offsets, row bases)
 // stay in scalar registers instead of being recomputed per lane.

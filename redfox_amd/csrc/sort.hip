@@ -1,11 +1,12 @@
-// sort.hip - stable LSD radix sort for gfx950: 8-bit digits (9 or 10 bits
-// when a context is tuned to them), one upfront histogram pass over the
-// keys for all digit positions, then one "onesweep" kernel per digit that
-// ranks a tile in registers/LDS, obtains its global digit offsets by
-// decoupled look-back and scatters through an LDS reorder buffer.  Wider
-// digits take fewer passes over the data (26-bit keys: 3 instead of 4;
-// 20-bit: 2 instead of 3) at the cost of more bins per tile: more ranking
-// ballots and look-back words, shorter runs per bin in the scatter.
+// sort.hip - stable LSD radix sort for gfx950: one upfront histogram pass
+// over the keys for all digit positions, then one "onesweep" kernel per
+// digit that ranks a tile in registers/LDS, obtains its global digit offsets
+// by decoupled look-back and scatters through an LDS reorder buffer.  Digits
+// are 8 bits, or 6 to 10 where key_bits makes an even number of passes of
+// them (auto_digit): wider digits take fewer passes over the data at the
+// cost of more bins per tile (more ranking ballots and look-back words,
+// shorter runs per bin in the scatter), narrower ones save the copy back
+// after an odd number of passes.
 //
 // Replaces redfox::sort_pair / sort_key (b40cSort.cu:58-1021: b40c LSD
 // radix, 4-5 bit digits, upsweep + spine + downsweep per digit, pong
@@ -26,36 +27,56 @@
 namespace rfx {
 namespace {
 
-// Digit width DB: 1 << DB bins.  8 by default; 9 and 10 for the
-// sort.digit knob.
+// Digit width DB: 1 << DB bins.
 template <int DB>
 constexpr int kBinsOf = 1 << DB;
 
-#ifndef RFX_SORT_NT
-#define RFX_SORT_NT 512
-#endif
-#ifndef RFX_SORT_IPT
-#define RFX_SORT_IPT 16
-#endif
-#ifndef RFX_SORT_MINW
-#define RFX_SORT_MINW 1
-#endif
-#ifndef RFX_SORT_LBW
-#define RFX_SORT_LBW 4
-#endif
-// Tile shape: NT threads x IPT keys per thread.  LDS per block is about
-// kMax*TILE (reorder) + TILE (digits) + 8 KB (wave counters): 16 keys per
-// thread for <= 4-byte elements, 14 for 8-byte (2 blocks per CU), 8 for
-// 16-byte.  (12 and 16 measure within 2% of each other on 2^28 u32 pairs,
-// in either order from box to box; the autotuner can pick 8, 12 or 16.)
-template <int KB, int VB>
+// Tile shape of the large sorts: NT threads x IPT keys per thread.  LDS per
+// block is about kMax*TILE (reorder) + 2*bins*NT/64 (wave counters) +
+// 4*bins.  The pass is bound by the cache lines that it writes in part, one
+// or two per tile, digit and column, so the tile is as large as the
+// registers allow with two blocks per CU (128 VGPRs; whole sorts of 2^28
+// u32 pairs: 512 x 16 4.81 ms, 512 x 20 4.74, 512 x 24 4.52, 512 x 32 4.65
+// with spills; 2^28 u32 keys alone: 512 x 16 1.81 ms at 2^27, 512 x 32
+// 1.62).  8-byte elements: two 512 x 14 blocks or, where the digits are 10
+// bits wide or keys and values are both 8 bytes, one block of 1024 (2^25
+// u32 keys of 20 bits with f64 values: 0.65 -> 0.57 ms; 2^26 u64 pairs
+// 3.97 -> 3.79 ms; u64 keys with u32 values 6.16 -> 7.1 ms, so not there).
+template <int KB, int VB, int DB>
 struct SortTune {
   static constexpr int kMax = KB > VB ? KB : VB;
-  static constexpr int NT = RFX_SORT_NT;
-  static constexpr int IPT = kMax >= 16 ? RFX_SORT_IPT / 2
-                             : kMax >= 8 ? (RFX_SORT_IPT * 7) / 8 : RFX_SORT_IPT;
-  static constexpr int TILE = NT * IPT;
+  static constexpr bool kWide = kMax == 8 && (DB == 10 || (KB == 8 && VB == 8));
+  static constexpr int NT = kWide ? 1024 : 512;
+  static constexpr int IPT = kMax >= 16             ? 8
+                             : kMax >= 8            ? (kWide && DB <= 8 ? 12 : 14)
+                             : KB == 4 && VB == 4   ? 24
+                             : KB == 4 && VB == 0   ? 32
+                                                    : 16;
 };
+
+// Look-back window (status words per round trip): every extra word polled
+// costs a large sort (2^28 u32 pairs 4.79 ms with 2, 4.81 with 4, 4.95 with
+// 8).
+constexpr int kWindow = 2;
+
+// Tile of the sorts whose large tiles would not fill the chip: kMidNT
+// threads x 4 keys (12 x 512 for 9 and 10 bit digits, whose counters fill
+// the LDS), up to kMidTiles such tiles per CU.  All of them run at once, and
+// their look-back goes by groups of tiles (kGroups) instead of a window.
+// 1 M u64 keys with u32 values: 178 us with tiles of 7168 and a window of
+// 4, 168 with tiles of 4096, 145 with groups as well.
+constexpr int kMidNT = 1024;
+constexpr int kMidIPT = 4;
+constexpr uint64_t kMidTiles = 2;
+constexpr int kGroups = 0;  // as a look-back window
+
+// Consecutive tiles that one XCD's queue takes at a time.  Fewer share fewer
+// lines; more keep the chunks after them waiting in their look-back (2^26
+// u64 pairs, tiles of 12288: 8 3.74 ms, 16 4.03; 2^27 u64 keys with u32
+// values, tiles of 7168: 8 6.20 ms, 16 6.10).
+template <int TILE>
+constexpr uint32_t kChunkOf = TILE >= 12288 ? 8 : 16;
+constexpr uint32_t kMinChunk = 8;
 
 // Look-back status words: 32 bits (2 flag bits, a 30-bit count) for up to
 // 2^30 - 1 rows, 64 bits (flags in bits 62-63) beyond, up to 2^31 - 1.
@@ -112,13 +133,134 @@ __device__ __forceinline__ uint32_t sort_lookback(const S* status, uint32_t tile
   }
 }
 
+// Hides x's value from the optimiser, so that what is computed from it
+// before is computed again afterwards instead of being kept in registers.
+template <class T>
+__device__ __forceinline__ void opaque(T& x) {
+  if constexpr (sizeof(T) <= 4) {
+    uint32_t t = x;
+    asm volatile("" : "+v"(t));
+    x = static_cast<T>(t);
+  } else if constexpr (sizeof(T) == 8) {
+    asm volatile("" : "+v"(x));
+  } else {
+    asm volatile("" : "+v"(x.lo), "+v"(x.hi));
+  }
+}
+
+// The same prefix when every tile of the sort runs at once: the tiles have
+// all published their aggregates and none has a prefix yet, so a walk back
+// reads most of them (1 M rows: 245 tiles, 10 us of an 18 us pass).  Instead
+// the last tile of each group of kGroup adds up its group's aggregates and
+// publishes the sum; a tile adds the aggregates before it in its group and
+// the sums of the groups before.  Tiles only wait for lower ones.
+constexpr uint32_t kGroup = 16;
+
+template <class S>
+__device__ __forceinline__ uint32_t sum_words(const S* p, uint32_t count, uint32_t stride) {
+  using SW = StatusWord<S>;
+  uint32_t sum = 0;
+  for (uint32_t i = 0; i < count; i += 8) {
+    S v[8];
+    bool all;
+    do {
+      all = true;
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j)
+        v[j] = i + j < count ? sw_load(p + static_cast<uint64_t>(i + j) * stride) : SW::kAgg;
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) all &= (v[j] & ~SW::kMask) != 0;
+    } while (!all);
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) sum += static_cast<uint32_t>(v[j] & SW::kMask);
+  }
+  return sum;
+}
+
+template <class S>
+__device__ __forceinline__ uint32_t sort_lookback_groups(const S* status, S* sums, uint32_t tile,
+                                                         uint32_t stride, uint32_t col,
+                                                         uint32_t own) {
+  using SW = StatusWord<S>;
+  const uint32_t g = tile / kGroup, in = tile % kGroup;
+  const uint32_t before =
+      sum_words(status + static_cast<uint64_t>(tile - in) * stride + col, in, stride);
+  if (in == kGroup - 1)
+    sw_store<S>(sums + static_cast<uint64_t>(g) * stride + col,
+                SW::kAgg | static_cast<S>(before + own));
+  return before + sum_words(sums + col, g, stride);
+}
+
+// ---- tiles -----------------------------------------------------------------
+// The pass's blocks are persistent and take tiles until none is left.  With
+// first == 0 every tile comes from one ticket.  Otherwise blocks are split
+// over kQueues queues by blockIdx, which the hardware deals out to the XCDs
+// in turn, and a queue hands out chunks of consecutive tiles (`first` tiles,
+// one for each of its blocks, then kChunk at a time): their runs of one
+// digit are neighbours in the output, so the cache lines that two tiles
+// share are completed in one XCD's L2 instead of being written twice, in
+// part, from two of them.
+//
+// A chunk's first tile (plus 1) is kept in the queue's list.  It comes from
+// the global ticket: chunk 0's with the queue's first tile, chunk k + 1's
+// with the first tile of chunk k, so that it is there when chunk k + 1
+// begins.  Whoever numbers chunk k + 1 has waited for chunk k's number, so
+// a queue's chunks are in increasing order.
+//
+// Progress: a queue hands out its tiles in increasing order, to any block of
+// the queue that is running, and a block exits only when its queue's next
+// chunk lies past the last tile.  So the lowest unfinished tile is either
+// held by a running block, whose predecessors are all done, or the next tile
+// of a queue whose blocks hold only lower tiles, all done: one of them takes
+// it.  Nothing depends on how many blocks are resident.
+constexpr uint32_t kQueues = 8;
+constexpr uint32_t kCtrLine = 32;  // words between counters (128 bytes)
+constexpr uint32_t kCtrWords = (2 + kQueues) * kCtrLine;
+
+// Chunks that one queue's list has room for: a queue that hands out all of
+// them, and the ones past the end that its blocks ask for.
+constexpr uint64_t queue_list(uint64_t tiles) { return tiles / kMinChunk + 4; }
+
+template <uint32_t kChunk>
+struct TileQueue {
+  uint32_t* ctr;   // [0] ticket, [kCtrLine] finished blocks, then the queues' counters
+  uint32_t* list;  // [kQueues][list_len]
+  uint32_t list_len;
+  uint32_t first;
+  // Ask for a tile (the answer is not waited for) ...
+  __device__ __forceinline__ uint32_t ask() const {
+    return atomicAdd(first ? ctr + (2 + blockIdx.x % kQueues) * kCtrLine : ctr, 1u);
+  }
+  // ... and the tile that the answer stands for (past the last one: none).
+  __device__ __forceinline__ uint32_t tile(uint32_t i) const {
+    if (!first) return i;
+    uint32_t* l = list + (blockIdx.x % kQueues) * list_len;
+    const uint32_t k = i < first ? 0 : 1 + (i - first) / kChunk;
+    const uint32_t in = i < first ? i : (i - first) % kChunk;
+    if (k >= list_len) return ~0u;
+    if (i == 0) sw_store(l, atomicAdd(ctr, first) + 1);
+    uint32_t t;
+    while ((t = sw_load(l + k)) == 0) __builtin_amdgcn_s_sleep(1);
+    if (in == 0 && k + 1 < list_len) sw_store(l + k + 1, atomicAdd(ctr, kChunk) + 1);
+    return t - 1 + in;
+  }
+};
+
+// Rows of status words of one pass: the tiles, then the groups of a sort
+// whose tiles all run at once.
+constexpr uint64_t kGroupedTiles = 2048;
+__host__ __device__ constexpr uint64_t status_rows(uint64_t tiles) {
+  return tiles + (tiles <= kGroupedTiles ? (tiles + kGroup - 1) / kGroup : 0);
+}
+
 struct SortLayout {
   uint32_t* hist;    // [P][bins]
   uint32_t* base;    // [P][bins] exclusive global digit offsets
-  uint32_t* ctrs;    // [P][2]   tile ticket, finished tiles
+  uint32_t* ctrs;    // [P][kCtrWords] tile queues
+  uint32_t* lists;   // [P][kQueues][queue_list(tiles)] their chunks
   uint32_t* skip;    // [P]
   uint32_t* sel;     // [1]      0: data in caller's buffers, 1: in pong
-  void* status;      // [P][tiles][bins] status words of S
+  void* status;      // [P][status_rows(tiles)][bins] status words of S
   void* pong_keys;
   void* pong_vals;
   uint64_t zero_words;  // words from hist to the end of status
@@ -127,10 +269,11 @@ struct SortLayout {
 static void carve_sort(Carve& c, uint64_t n, int kb, int vb, int passes, uint64_t tiles,
                        uint32_t bins, SortLayout* L, bool wide = false) {
   // The zeroed block comes first so it is one contiguous range.
-  const uint64_t status_words = static_cast<uint64_t>(passes) * tiles * bins;
+  const uint64_t status_words = static_cast<uint64_t>(passes) * status_rows(tiles) * bins;
   L->hist = c.take<uint32_t>(static_cast<uint64_t>(passes) * bins);
   L->base = c.take<uint32_t>(static_cast<uint64_t>(passes) * bins);
-  L->ctrs = c.take<uint32_t>(static_cast<uint64_t>(passes) * 2);
+  L->ctrs = c.take<uint32_t>(static_cast<uint64_t>(passes) * kCtrWords);
+  L->lists = c.take<uint32_t>(static_cast<uint64_t>(passes) * kQueues * queue_list(tiles));
   L->skip = c.take<uint32_t>(static_cast<uint64_t>(passes));
   L->sel = c.take<uint32_t>(1);
   L->status = wide ? static_cast<void*>(c.take<uint64_t>(status_words))
@@ -161,19 +304,26 @@ __device__ __forceinline__ uint32_t dig(K k, uint32_t shift, uint32_t m) {
 }
 
 // Histogram of every digit position in one read of the keys.  With an
-// aligned key pointer each thread reads 16 bytes at a time.
+// aligned key pointer each thread reads 16 bytes at a time.  Blocks are
+// large and few, since each adds its bins to the global ones by atomics
+// (1 M u64 keys: 245 blocks of 256 threads 18.7 us, mostly those adds).  The
+// last block to finish scans every digit's bins into offsets and flags the
+// identity passes.
+constexpr int kHistNT = 1024;
 template <int KB, bool VEC, int DB>
-__global__ __launch_bounds__(256) void k_radix_hist(const typename Elem<KB>::T* __restrict__ keys,
-                                                    uint64_t n, int passes, uint32_t key_bits,
-                                                    uint32_t* __restrict__ hist) {
+__global__ __launch_bounds__(kHistNT) void k_radix_hist(
+    const typename Elem<KB>::T* __restrict__ keys, uint64_t n, int passes, uint32_t key_bits,
+    uint32_t* __restrict__ hist, uint32_t* __restrict__ base, uint32_t* __restrict__ skip,
+    uint32_t* __restrict__ finished) {
   using K = typename Elem<KB>::T;
   constexpr int kBins = kBinsOf<DB>;
   constexpr int PER = (VEC && KB < 16) ? 16 / KB : 1;
+  __shared__ bool s_last;
   __shared__ uint32_t lh[(8 * KB + DB - 1) / DB * kBins];
-  for (int i = threadIdx.x; i < passes * kBins; i += 256) lh[i] = 0;
+  for (int i = threadIdx.x; i < passes * kBins; i += kHistNT) lh[i] = 0;
   __syncthreads();
-  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * 256;
-  const uint64_t gtid = blockIdx.x * 256ull + threadIdx.x;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kHistNT;
+  const uint64_t gtid = blockIdx.x * static_cast<uint64_t>(kHistNT) + threadIdx.x;
   auto count = [&](K k) {
     for (int p = 0; p < passes; ++p)
       atomicAdd(&lh[p * kBins + dig<DB>(k, DB * p, pass_mask<DB>(p, key_bits))], 1u);
@@ -215,34 +365,46 @@ __global__ __launch_bounds__(256) void k_radix_hist(const typename Elem<KB>::T* 
   }
   for (uint64_t i = done + gtid; i < n; i += stride) count(keys[i]);
   __syncthreads();
-  for (int i = threadIdx.x; i < passes * kBins; i += 256)
-    if (lh[i]) atomicAdd(&hist[i], lh[i]);
+  // The adds' old values are waited for, so a block counts as finished only
+  // when its adds are done (a release fence would write the whole L2 back,
+  // in every wave: 12 M keys 0.30 -> 0.36 ms).
+  uint32_t old = 0;
+  for (int i = threadIdx.x; i < passes * kBins; i += kHistNT)
+    if (lh[i]) old |= atomicAdd(&hist[i], lh[i]);
+  asm volatile("" ::"v"(old) : "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = atomicAdd(finished, 1u) == gridDim.x - 1;
+  __syncthreads();
+  if (!s_last) return;
+  // One wave per digit, kBins / 64 consecutive bins per lane.
+  constexpr int PL = kBins / kWave;
+  for (int p = static_cast<int>(wave_id()); p < passes; p += kHistNT / kWave) {
+    const uint32_t at = p * kBins + lane_id() * PL;
+    uint32_t c[PL], sum = 0;
+    bool one = false;  // every key has the same digit here
+#pragma unroll
+    for (int j = 0; j < PL; ++j) {
+      c[j] = sw_load(hist + at + j);
+      sum += c[j];
+      one |= c[j] == n;
+    }
+    uint32_t run = wave_incl_scan(sum) - sum;
+#pragma unroll
+    for (int j = 0; j < PL; ++j) {
+      base[at + j] = run;
+      run += c[j];
+    }
+    if (one) skip[p] = 1u;  // at most one lane: the bins add up to n
+  }
 }
 
-// Exclusive scan of each digit histogram (one thread per bin); flags
-// identity passes.
-template <int DB>
-__global__ __launch_bounds__(kBinsOf<DB>) void k_radix_scan(const uint32_t* __restrict__ hist,
-                                                            uint32_t* __restrict__ base,
-                                                            uint32_t* __restrict__ skip,
-                                                            uint64_t n) {
-  constexpr int kBins = kBinsOf<DB>;
-  __shared__ uint32_t tmp[kBins / kWave + 1];
-  const int p = blockIdx.x;
-  const uint32_t c = hist[p * kBins + threadIdx.x];
-  uint32_t total;
-  uint32_t e = block_excl_scan<kBins>(c, tmp, &total);
-  base[p * kBins + threadIdx.x] = e;
-  if (c == n) skip[p] = 1u;  // every key has the same digit here
-}
-
-template <int KB, int VB, int NT, int IPT, int DB, class S>
-__global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
+template <int KB, int VB, int NT, int IPT, int DB, int LBW, class S>
+__global__ __launch_bounds__(NT, 4) void k_onesweep(
     typename Elem<KB>::T* __restrict__ k0, typename Elem<KB>::T* __restrict__ k1,
     typename Elem<VB>::T* __restrict__ v0, typename Elem<VB>::T* __restrict__ v1, uint64_t n,
     int pass, uint32_t key_bits, const uint32_t* __restrict__ base, uint32_t* __restrict__ ctrs,
     const uint32_t* __restrict__ skip, uint32_t* __restrict__ sel, S* __restrict__ status,
-    uint32_t ntiles) {
+    uint32_t ntiles, uint32_t first, uint32_t* __restrict__ lists, uint32_t list_len) {
   using K = typename Elem<KB>::T;
   using V = typename Elem<VB>::T;
   constexpr int NW = NT / kWave;
@@ -250,11 +412,12 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
   constexpr int RB = (KB > VB ? KB : VB) * TILE;
   constexpr int kBins = kBinsOf<DB>;
   constexpr int BPT = (kBins + NT - 1) / NT;  // bins per thread in the per-bin steps
+  constexpr int NBW = (kBins < NT ? kBins : NT) / kWave;  // waves that hold bins
+  constexpr int kScatterBatch = 8;  // scattered at a time: bounds the registers in flight
   // Wave counters and tile positions stay below TILE: 16 bits hold them,
   // which keeps the wider digits' counters within LDS.
-  using WC = typename std::conditional<(DB > 8), uint16_t, uint32_t>::type;
-  using DG = typename std::conditional<(DB > 8), uint16_t, uint8_t>::type;
-  static_assert(TILE <= 65535 || DB == 8, "16-bit wave counters");
+  using WC = uint16_t;
+  static_assert(TILE <= 65535 && IPT % 2 == 0, "16-bit wave counters, packed positions");
 
   if (skip[pass]) return;
   const uint32_t cur = *sel;
@@ -264,31 +427,28 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
   V* __restrict__ vout = cur ? v0 : v1;
 
   __shared__ uint32_t s_tile;
-  __shared__ WC wcnt[NW][kBins];
+  __shared__ __attribute__((aligned(16))) WC wcnt[NW][kBins];
   __shared__ uint32_t gdelta[kBins];
-  __shared__ uint32_t scan_tmp[NW + 1];
+  __shared__ uint32_t s_scan[BPT][NBW];
   __shared__ __attribute__((aligned(16))) unsigned char rbuf[RB];
-  __shared__ DG sdig[VB > 0 ? TILE : 1];  // digit of each reordered row
 
-  const uint32_t tid = threadIdx.x;
-  const uint32_t lane = lane_id();
-  const uint32_t w = wave_id();
+  const uint32_t n32 = static_cast<uint32_t>(n);
   const uint32_t shift = static_cast<uint32_t>(DB * pass);
   const uint32_t dmask = pass_mask<DB>(pass, key_bits);
 
-  if (tid == 0) s_tile = atomicAdd(&ctrs[pass * 2], 1u);
-  for (uint32_t i = tid; i < NW * kBins; i += NT) (&wcnt[0][0])[i] = 0;
-  __syncthreads();
-  const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);  // block-uniform: scalar from here
-  const uint64_t tile_base = static_cast<uint64_t>(tile) * TILE;
-  const uint64_t wave_base = tile_base + static_cast<uint64_t>(w) * kWave * IPT;
+  uint32_t tid = threadIdx.x, lane = lane_id();
+  const uint32_t w = wave_id();
+  const TileQueue<kChunkOf<TILE>> queue{ctrs + pass * kCtrWords, lists + pass * kQueues * list_len, list_len, first};
+  if (tid == 0) s_tile = queue.tile(queue.ask());
   using SW = StatusWord<S>;
-  S* st = status + (static_cast<uint64_t>(pass) * ntiles) * kBins;
+  S* st = status + (static_cast<uint64_t>(pass) * status_rows(ntiles)) * kBins;
 
   // Every tile but the last is full: its copy of the body has no per-key
   // bounds checks.
-  auto body = [&](auto full_tag) {
+  auto body = [&](uint32_t tile, auto full_tag) {
     constexpr bool FULL = decltype(full_tag)::value;
+    const uint64_t tile_base = static_cast<uint64_t>(tile) * TILE;
+    const uint64_t wave_base = tile_base + static_cast<uint64_t>(w) * kWave * IPT;
     // Keys only: values are read after the keys are ranked, which keeps
     // the ranking phase's register footprint small.
     K keys[IPT];
@@ -304,7 +464,7 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
     // (An LDS atomic per group leader, issued for all keys before any
     // result is used, measured slower on MI355X: 1.67 against 1.45 ms per
     // pass.)
-    uint32_t pos[IPT];
+    uint32_t pos[IPT / 2];
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
       const uint64_t idx = wave_base + static_cast<uint64_t>(j) * kWave + lane;
@@ -335,10 +495,16 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
         prior = wcnt[w][d];
         if (below == cnt - 1) wcnt[w][d] = static_cast<WC>(prior + cnt);
       }
-      pos[j] = prior + below;
+      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t r = prior + below;
+      pos[j / 2] = (j & 1) ? (pos[j / 2] | (r << 16)) : r;
     }
     __syncthreads();
 
+    // The digits and counter addresses of the ranking are not kept (90 -> 80
+    // registers at 16 keys).
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) opaque(keys[j]);
     // Per-digit tile totals and wave prefixes; publish the tile aggregate.
     // wcnt[w][d] becomes the tile position of wave w's first key of digit
     // d: the digit's start in the tile plus the waves before w.
@@ -362,12 +528,27 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
                     (tile == 0 ? SW::kIncl : SW::kAgg) | static_cast<S>(run));
       }
     }
+    // Each digit's start in the tile: scans within the waves, then the
+    // totals of the waves before.
+#pragma unroll
+    for (int q = 0; q < BPT; ++q) {
+      const uint32_t incl = wave_incl_scan(total_d[q]);
+      if (w < NBW && lane == kWave - 1) s_scan[q][w] = incl;
+      bs[q] = incl - total_d[q];
+    }
+    __syncthreads();
     {
       uint32_t carry = 0;
 #pragma unroll
       for (int q = 0; q < BPT; ++q) {
-        uint32_t all;
-        bs[q] = carry + block_excl_scan<NT>(total_d[q], scan_tmp, &all);
+        uint32_t all = 0;
+#pragma unroll
+        for (int i = 0; i < NBW; ++i) {
+          const uint32_t x = s_scan[q][i];
+          bs[q] += static_cast<uint32_t>(i) < w ? x : 0u;
+          all += x;
+        }
+        bs[q] += carry;
         carry += all;
       }
     }
@@ -390,8 +571,10 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
       const uint64_t idx = wave_base + static_cast<uint64_t>(j) * kWave + lane;
       if (FULL || idx < n) {
         const uint32_t d = dig<DB>(keys[j], shift, dmask);
-        pos[j] += wcnt[w][d];
-        kbuf[pos[j]] = keys[j];
+        const uint32_t off = wcnt[w][d];
+        const uint32_t at = ((j & 1) ? (pos[j / 2] >> 16) : (pos[j / 2] & 0xFFFFu)) + off;
+        pos[j / 2] += (j & 1) ? (off << 16) : off;
+        kbuf[at] = keys[j];
       }
     }
     V vals[IPT];
@@ -407,8 +590,11 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
       const uint32_t bin = tid + q * NT;
       if (bin < kBins) {
         uint32_t excl = 0;
-        if (tile > 0) {
-          excl = sort_lookback<RFX_SORT_LBW>(st, tile, kBins, bin);
+        if constexpr (LBW == kGroups) {
+          excl = sort_lookback_groups<S>(st, st + static_cast<uint64_t>(ntiles) * kBins, tile,
+                                         kBins, bin, total_d[q]);
+        } else if (tile > 0) {
+          excl = sort_lookback<LBW>(st, tile, kBins, bin);
           sw_store<S>(st + static_cast<uint64_t>(tile) * kBins + bin,
                       SW::kIncl | static_cast<S>(excl + total_d[q]));
         }
@@ -420,16 +606,22 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
     const uint32_t tile_n =
         FULL ? static_cast<uint32_t>(TILE)
              : static_cast<uint32_t>((n - tile_base) < TILE ? (n - tile_base) : TILE);
+    uint32_t dst[IPT];
 #pragma unroll
     for (int k = 0; k < IPT; ++k) {
+      if (k % kScatterBatch == 0) __builtin_amdgcn_sched_barrier(0);
       const uint32_t i = k * NT + tid;
       if (FULL || i < tile_n) {
         const K key = kbuf[i];
         const uint32_t d = dig<DB>(key, shift, dmask);
-        if constexpr (VB > 0) sdig[i] = static_cast<DG>(d);
-        const uint32_t dst = gdelta[d] + i;
-        if (dst < n) kout[dst] = key;  // always true when ranks are right
+        dst[k] = gdelta[d] + i;
+        if (dst[k] < n32) kout[dst[k]] = key;  // always true when ranks are right
       }
+    }
+    // The next tile is asked for while this one is still being stored.
+    uint32_t next = 0;
+    if constexpr (VB == 0) {
+      if (tid == 0) s_tile = queue.tile(queue.ask());
     }
     if constexpr (VB > 0) {
       __syncthreads();  // every key is out of kbuf
@@ -437,27 +629,40 @@ __global__ __launch_bounds__(NT, RFX_SORT_MINW) void k_onesweep(
 #pragma unroll
       for (int j = 0; j < IPT; ++j) {
         const uint64_t idx = wave_base + static_cast<uint64_t>(j) * kWave + lane;
-        if (FULL || idx < n) vbuf[pos[j]] = vals[j];
+        if (FULL || idx < n) vbuf[(j & 1) ? (pos[j / 2] >> 16) : (pos[j / 2] & 0xFFFFu)] = vals[j];
       }
       __syncthreads();
+      if (tid == 0) next = queue.ask();
 #pragma unroll
       for (int k = 0; k < IPT; ++k) {
+        if (k % kScatterBatch == 0) __builtin_amdgcn_sched_barrier(0);
         const uint32_t i = k * NT + tid;
         if (FULL || i < tile_n) {
-          const uint32_t dst = gdelta[sdig[i]] + i;
-          if (dst < n) vout[dst] = vbuf[i];
+          if (dst[k] < n32) vout[dst[k]] = vbuf[i];
         }
       }
+      if (tid == 0) s_tile = queue.tile(next);
     }
   };
-  if (tile_base + TILE <= n) body(std::true_type{});
-  else body(std::false_type{});
+  for (;;) {
+    // Opaque to the compiler in each round: addresses made of them are
+    // worked out where they are used, not kept in registers around the loop.
+    opaque(tid);
+    opaque(lane);
+    for (uint32_t i = tid; i < NW * kBins / 2; i += NT)
+      reinterpret_cast<uint32_t*>(&wcnt[0][0])[i] = 0;
+    __syncthreads();
+    const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);  // block-uniform: scalar from here
+    if (tile >= ntiles) break;
+    if (static_cast<uint64_t>(tile) * TILE + TILE <= n) body(tile, std::true_type{});
+    else body(tile, std::false_type{});
+  }
 
-  // The last tile to finish flips the buffer selector.  Every block read
+  // The last block to finish flips the buffer selector.  Every block read
   // *sel before arriving here, so nobody reads the new value this pass.
   if (tid == 0) {
-    const uint32_t prev = atomicAdd(&ctrs[pass * 2 + 1], 1u);
-    if (prev == ntiles - 1)
+    const uint32_t prev = atomicAdd(&queue.ctr[kCtrLine], 1u);
+    if (prev == gridDim.x - 1)
       __hip_atomic_store(sel, cur ^ 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -476,11 +681,13 @@ __global__ __launch_bounds__(256) void k_copyback(typename Elem<KB>::T* __restri
   }
 }
 
-// Tunable tile shapes: the autotuner may pick 8, 12 or 16 keys per thread for
-// 4- and 8-byte keys with 0-, 4- or 8-byte values (other shapes keep the
-// default).  The smallest tile needs the most look-back status words.
+// Tunable tile shapes: the autotuner may pick 8, 12 or 16 keys per thread
+// (of 512) for 4- and 8-byte keys with 0-, 4- or 8-byte values; other shapes
+// keep the default.  The smallest tile needs the most look-back status
+// words.
 template <int KB, int VB>
 constexpr bool kSortTunable = (KB == 4 || KB == 8) && (VB == 0 || VB == 4 || VB == 8);
+constexpr int kTuneNT = 512;
 constexpr int kSortMinIPT = 8;
 
 uint64_t sort_ws_tile(uint64_t n, int kb, int vb, int key_bits, uint64_t tile, int db,
@@ -504,8 +711,15 @@ constexpr uint64_t kSortMaxRows = (1ull << 31) - 1;
 // pairs, 18 bits 3.36 ms against 5.04, 20 bits 4.04 against 4.90.  Wider
 // keys keep 8 bits (26 bits: 5.51 ms against 5.65 with 9; 32 bits: 5.56
 // against 6.29).
+// 21-24 bit keys take four passes of 6 bits instead of three of 8 and the
+// copy, 25-28 bit keys four of 7 bits: fewer bins per tile, so fewer lines
+// written in part.
 constexpr int auto_digit(int key_bits) {
-  return key_bits >= 17 && key_bits <= 18 ? 9 : key_bits >= 19 && key_bits <= 20 ? 10 : 8;
+  return key_bits >= 17 && key_bits <= 18   ? 9
+         : key_bits >= 19 && key_bits <= 20 ? 10
+         : key_bits >= 21 && key_bits <= 24 ? 6
+         : key_bits >= 25 && key_bits <= 28 ? 7
+                                            : 8;
 }
 
 // Workspace for any tile shape the context may be tuned to, at the digit
@@ -513,26 +727,25 @@ constexpr int auto_digit(int key_bits) {
 // its own workspace on first use).
 template <int KB, int VB>
 uint64_t sort_ws_bytes(uint64_t n, int key_bits) {
-  using Tn = SortTune<KB, VB>;
-  const int ipt = kSortTunable<KB, VB> && kSortMinIPT < Tn::IPT ? kSortMinIPT : Tn::IPT;
-  if (n > kCountMask)
-    return sort_ws_tile(n, KB, VB, key_bits, static_cast<uint64_t>(Tn::NT) * Tn::IPT, 8, true);
-  uint64_t ws = sort_ws_tile(n, KB, VB, key_bits, static_cast<uint64_t>(Tn::NT) * ipt, 8);
+  using Tn = SortTune<KB, VB, 8>;
+  const uint64_t tile = static_cast<uint64_t>(Tn::NT) * Tn::IPT;
+  if (n > kCountMask) return sort_ws_tile(n, KB, VB, key_bits, tile, 8, true);
+  constexpr uint64_t kMinTile = kTuneNT * kSortMinIPT;
+  uint64_t ws = sort_ws_tile(n, KB, VB, key_bits,
+                             kSortTunable<KB, VB> && kMinTile < tile ? kMinTile : tile, 8);
   if (kSortTunable<KB, VB> && auto_digit(key_bits) != 8) {
-    const int wide_ipt = Tn::IPT < 12 ? Tn::IPT : 12;
     const uint64_t w2 = sort_ws_tile(n, KB, VB, key_bits,
-                                     static_cast<uint64_t>(Tn::NT) * wide_ipt,
+                                     auto_digit(key_bits) > 8 ? kTuneNT * 12ull : kMinTile,
                                      auto_digit(key_bits));
     if (w2 > ws) ws = w2;
   }
   return ws;
 }
 
-template <int KB, int VB, int IPT, int DB = 8, class S = uint32_t>
+template <int KB, int VB, int NT, int IPT, int DB, int LBW = kWindow, class S = uint32_t>
 int sort_impl(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
   using K = typename Elem<KB>::T;
   using V = typename Elem<VB>::T;
-  constexpr int NT = SortTune<KB, VB>::NT;
   constexpr int TILE = NT * IPT;
   constexpr bool kWide = sizeof(S) == 8;
   if (n < 2) return RFX_OK;
@@ -547,28 +760,40 @@ int sort_impl(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
   carve_sort(c, n, KB, VB, passes, tiles, kBins, &L, kWide);
   RFX_TRY(fill_u32(ctx, L.hist, L.zero_words, 0u));
 
-  uint64_t hb = (n + 256 * 16 - 1) / (256 * 16);
-  uint64_t hmax = static_cast<uint64_t>(ctx->device_cus) * 8;
+  constexpr uint64_t kHistRows = kHistNT * 16;  // per block
+  uint64_t hb = (n + kHistRows - 1) / kHistRows;
+  const uint64_t hmax = static_cast<uint64_t>(ctx->device_cus) * 2;
   if (hb > hmax) hb = hmax;
-  if (hb == 0) hb = 1;
   {
     RFX_PROF(ctx, "sort.hist");
     if (reinterpret_cast<uintptr_t>(keys) % 16 == 0)
-      k_radix_hist<KB, true, DB><<<static_cast<uint32_t>(hb), 256, 0, ctx->stream>>>(
-          static_cast<const K*>(keys), n, passes, static_cast<uint32_t>(key_bits), L.hist);
+      k_radix_hist<KB, true, DB><<<static_cast<uint32_t>(hb), kHistNT, 0, ctx->stream>>>(
+          static_cast<const K*>(keys), n, passes, static_cast<uint32_t>(key_bits), L.hist, L.base,
+          L.skip, L.ctrs + 1);
     else
-      k_radix_hist<KB, false, DB><<<static_cast<uint32_t>(hb), 256, 0, ctx->stream>>>(
-          static_cast<const K*>(keys), n, passes, static_cast<uint32_t>(key_bits), L.hist);
+      k_radix_hist<KB, false, DB><<<static_cast<uint32_t>(hb), kHistNT, 0, ctx->stream>>>(
+          static_cast<const K*>(keys), n, passes, static_cast<uint32_t>(key_bits), L.hist, L.base,
+          L.skip, L.ctrs + 1);
     RFX_LAUNCHED();
   }
-  k_radix_scan<DB><<<passes, kBins, 0, ctx->stream>>>(L.hist, L.base, L.skip, n);
-  RFX_LAUNCHED();
+  static const int per_cu = [] {
+    int b = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &b, reinterpret_cast<const void*>(k_onesweep<KB, VB, NT, IPT, DB, LBW, S>), NT, 0) !=
+            hipSuccess || b < 1)
+      b = 1;
+    return b;
+  }();
+  const uint64_t slots = static_cast<uint64_t>(ctx->device_cus) * per_cu;
+  const uint32_t grid = static_cast<uint32_t>(tiles < slots ? tiles : slots);
+  const uint32_t first = tiles > 2 * slots ? (grid + kQueues - 1) / kQueues : 0;
   for (int p = 0; p < passes; ++p) {
     RFX_PROF(ctx, "sort.onesweep");
-    k_onesweep<KB, VB, NT, IPT, DB, S><<<static_cast<uint32_t>(tiles), NT, 0, ctx->stream>>>(
+    k_onesweep<KB, VB, NT, IPT, DB, LBW, S><<<grid, NT, 0, ctx->stream>>>(
         static_cast<K*>(keys), static_cast<K*>(L.pong_keys), static_cast<V*>(vals),
         static_cast<V*>(L.pong_vals), n, p, static_cast<uint32_t>(key_bits), L.base, L.ctrs,
-        L.skip, L.sel, static_cast<S*>(L.status), static_cast<uint32_t>(tiles));
+        L.skip, L.sel, static_cast<S*>(L.status), static_cast<uint32_t>(tiles), first, L.lists,
+        static_cast<uint32_t>(queue_list(tiles)));
     RFX_LAUNCHED();
   }
   uint64_t cb = (n + 255) / 256;
@@ -580,28 +805,44 @@ int sort_impl(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
   return RFX_OK;
 }
 
+// At one digit width: the large tile, or for a sort whose large tiles would
+// not fill the chip, a small one.
+template <int KB, int VB, int DB>
+int sort_digits(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
+  using Tn = SortTune<KB, VB, DB>;
+  constexpr int NT = DB > 8 ? kTuneNT : kMidNT, IPT = DB > 8 ? 12 : kMidIPT;
+  if constexpr (kSortTunable<KB, VB>) {
+    if (n <= ctx->device_cus * kMidTiles * NT * IPT)
+      return sort_impl<KB, VB, NT, IPT, DB, kGroups>(ctx, keys, vals, n, key_bits);
+  }
+  return sort_impl<KB, VB, Tn::NT, Tn::IPT, DB>(ctx, keys, vals, n, key_bits);
+}
+
 template <int KB, int VB>
 int sort_tuned(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
+  using Tn = SortTune<KB, VB, 8>;
   // More than 2^30 - 1 rows (or the sort.status knob at 64): 64-bit status
   // words, default tile, 8-bit digits.
   if (n > kCountMask || ctx->tune_sort_status == 64)
-    return sort_impl<KB, VB, SortTune<KB, VB>::IPT, 8, uint64_t>(ctx, keys, vals, n, key_bits);
+    return sort_impl<KB, VB, Tn::NT, Tn::IPT, 8, kWindow, uint64_t>(ctx, keys, vals, n,
+                                                                         key_bits);
   if constexpr (kSortTunable<KB, VB>) {
-    // Wider digits: the default tile, or 12 keys per thread.  Knob value 0
-    // takes the digit width chosen for key_bits.
-    constexpr int D = SortTune<KB, VB>::IPT;
+    // Knob value 0 takes the digit width chosen for key_bits.
     const int digit = ctx->tune_sort_digit ? ctx->tune_sort_digit : auto_digit(key_bits);
+    const int ipt = ctx->tune_sort_ipt;
+    if (digit == 6) return sort_digits<KB, VB, 6>(ctx, keys, vals, n, key_bits);
+    if (digit == 7) return sort_digits<KB, VB, 7>(ctx, keys, vals, n, key_bits);
     if (digit == 9)
-      return ctx->tune_sort_ipt == 12 ? sort_impl<KB, VB, 12, 9>(ctx, keys, vals, n, key_bits)
-                                      : sort_impl<KB, VB, D, 9>(ctx, keys, vals, n, key_bits);
+      return ipt == 12 ? sort_impl<KB, VB, kTuneNT, 12, 9>(ctx, keys, vals, n, key_bits)
+                       : sort_digits<KB, VB, 9>(ctx, keys, vals, n, key_bits);
     if (digit == 10)
-      return ctx->tune_sort_ipt == 12 ? sort_impl<KB, VB, 12, 10>(ctx, keys, vals, n, key_bits)
-                                      : sort_impl<KB, VB, D, 10>(ctx, keys, vals, n, key_bits);
-    if (ctx->tune_sort_ipt == 8) return sort_impl<KB, VB, 8>(ctx, keys, vals, n, key_bits);
-    if (ctx->tune_sort_ipt == 12) return sort_impl<KB, VB, 12>(ctx, keys, vals, n, key_bits);
-    if (ctx->tune_sort_ipt == 16) return sort_impl<KB, VB, 16>(ctx, keys, vals, n, key_bits);
+      return ipt == 12 ? sort_impl<KB, VB, kTuneNT, 12, 10>(ctx, keys, vals, n, key_bits)
+                       : sort_digits<KB, VB, 10>(ctx, keys, vals, n, key_bits);
+    if (ipt == 8) return sort_impl<KB, VB, kTuneNT, 8, 8>(ctx, keys, vals, n, key_bits);
+    if (ipt == 12) return sort_impl<KB, VB, kTuneNT, 12, 8>(ctx, keys, vals, n, key_bits);
+    if (ipt == 16) return sort_impl<KB, VB, kTuneNT, 16, 8>(ctx, keys, vals, n, key_bits);
   }
-  return sort_impl<KB, VB, SortTune<KB, VB>::IPT>(ctx, keys, vals, n, key_bits);
+  return sort_digits<KB, VB, 8>(ctx, keys, vals, n, key_bits);
 }
 
 template <int KB>

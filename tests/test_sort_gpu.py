@@ -225,3 +225,25 @@ def test_more_than_2p30_rows_properties(rf, ctx):
     seen = np.zeros(n, dtype=bool)
     seen[v] = True
     assert seen.all()
+
+
+# Past 2 x 256 CUs x 2 blocks of the largest tile, where tiles are handed out
+# by the XCDs' queues; the last size of the small tiles and the next; group
+# and tile edges of the small tiles; even and odd numbers of 6 and 7 bit
+# digits (a skipped pass included).
+@pytest.mark.parametrize("kb,vb,bits,n", [
+    (4, 4, 32, 12_582_912 + 12_289), (4, 0, 32, 16_777_216 + 1), (8, 4, 64, 7_340_032 + 77),
+    (8, 8, 24, 6_291_456 + 12_287), (4, 8, 20, 7_340_032 + 14_337),
+    (4, 4, 32, 2_097_152), (4, 4, 32, 2_097_153), (4, 8, 18, 3_145_729),
+    (8, 0, 64, 65_536), (8, 8, 64, 65_537), (4, 4, 23, 4_096 * 15), (4, 4, 21, 4_096 * 32 + 1),
+    (4, 4, 27, 5_000_001), (8, 4, 25, 4_097), (4, 4, 28, 2_500_000), (8, 0, 22, 3_000_003)])
+def test_tile_queues_and_small_tiles_match_numpy(rf, ctx, kb, vb, bits, n):
+    keys = make(kb, n, 1000 + bits) & DT[kb]((1 << bits) - 1 if bits < 64 else -1 % (1 << 64))
+    if bits == 27:
+        keys &= DT[kb](0x7F03FFF)  # the third 7-bit digit is zero: its pass is skipped
+    vals = make(vb, n, 1001) if vb else None
+    gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gk, keys[order])
+    if vb:
+        assert np.array_equal(gv, vals[order])
