@@ -398,6 +398,156 @@ __global__ __launch_bounds__(kHistNT) void k_radix_hist(
   }
 }
 
+// The lanes whose digit is this lane's.  acc collects, per lane, the lanes
+// whose digit differs in some bit: x is the lane's bit b as 0 or all ones,
+// and acc | (bb ^ x) is one bitop3 per 32-bit half (table 0xDE with acc in
+// the middle operand is the same under either operand order of the truth
+// table).  Bits above a narrow last digit are zero everywhere and change
+// nothing.
+template <int DB>
+__device__ __forceinline__ uint64_t same_digit(uint32_t d) {
+  uint32_t acc_lo = 0, acc_hi = 0;
+#pragma unroll
+  for (int b = 0; b < DB; ++b) {
+    const uint32_t x = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(d), b, 1));
+    // The ballot of x itself (a plain ballot(x != 0) is rewritten into a
+    // second shift-and-compare of d); 33 is the not-equal predicate.  Lanes
+    // outside exec give 0, as a ballot does.
+    const uint64_t bb = __builtin_amdgcn_uicmp(x, 0u, 33);
+    acc_lo = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(bb), acc_lo, x, 0xDE);
+    acc_hi = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(bb >> 32), acc_hi, x, 0xDE);
+  }
+  return ~((static_cast<uint64_t>(acc_hi) << 32) | acc_lo);
+}
+
+// A whole sort in one block: rows in registers, every pass's exchange
+// through LDS.  Seven launches and the trips of a look-back are what a small
+// sort costs otherwise (u32 pairs, the call alone: 1,000 rows 35 -> 11 us,
+// 4,099 39 -> 20, 8,000 45 -> 27; past that one CU takes longer than the
+// passes do).  Digits in which no two keys differ are left out.
+constexpr int kBlockNT = 1024;
+template <int KB, int VB>
+constexpr int kBlockIPT = (KB > VB ? KB : VB) >= 16 ? 4 : 8;
+
+template <int KB, int VB>
+__global__ __launch_bounds__(kBlockNT) void k_sort_block(typename Elem<KB>::T* __restrict__ keys,
+                                                         typename Elem<VB>::T* __restrict__ vals,
+                                                         uint32_t n, uint32_t key_bits) {
+  using K = typename Elem<KB>::T;
+  using V = typename Elem<VB>::T;
+  constexpr int IPT = kBlockIPT<KB, VB>;
+  constexpr int NW = kBlockNT / kWave, kBins = 256, NBW = kBins / kWave;
+  __shared__ __attribute__((aligned(16))) K kbuf[kBlockNT * IPT];
+  __shared__ __attribute__((aligned(16))) V vbuf[VB > 0 ? kBlockNT * IPT : 1];
+  __shared__ __attribute__((aligned(16))) uint16_t wcnt[NW][kBins];
+  __shared__ uint32_t s_scan[NBW];
+  __shared__ uint32_t s_vary[4];  // bits in which some key differs from the first
+  const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
+  // Wave w holds rows w*64*ipt .. of the present order, 64 to a step.
+  const uint32_t ipt = (n + kBlockNT - 1) / kBlockNT;
+  const uint32_t row0 = w * ipt * kWave + lane;
+  if (tid < 4) s_vary[tid] = 0;
+  const K first = keys[0];
+  K k[IPT];
+  V v[IPT];
+  u128 vary{0, 0};
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const uint32_t i = row0 + j * kWave;
+    if (static_cast<uint32_t>(j) < ipt && i < n) {
+      k[j] = keys[i];
+      if constexpr (VB > 0) v[j] = vals[i];
+      const u128 a = to128(k[j]), b = to128(first);
+      vary.lo |= a.lo ^ b.lo;
+      if constexpr (KB == 16) vary.hi |= a.hi ^ b.hi;
+    }
+  }
+  __syncthreads();
+  {
+    const uint32_t words[4] = {static_cast<uint32_t>(vary.lo), static_cast<uint32_t>(vary.lo >> 32),
+                               static_cast<uint32_t>(vary.hi), static_cast<uint32_t>(vary.hi >> 32)};
+#pragma unroll
+    for (int q = 0; q < (KB + 3) / 4; ++q) {
+      uint32_t x = words[q];
+#pragma unroll
+      for (int d = kWave / 2; d > 0; d >>= 1) x |= __shfl_xor(x, d, kWave);
+      if (lane == 0 && x) atomicOr(&s_vary[q], x);
+    }
+  }
+  for (uint32_t shift = 0; shift < key_bits; shift += 8) {
+    const uint32_t dmask = key_bits - shift < 8 ? (1u << (key_bits - shift)) - 1u : 0xFFu;
+    __syncthreads();  // the last exchange is read (before the first digit: s_vary is written)
+    if (!((s_vary[shift / 32] >> (shift % 32)) & dmask)) continue;  // uniform
+#pragma unroll
+    for (int q = 0; q < NW * kBins / 2 / kBlockNT; ++q)
+      reinterpret_cast<uint32_t*>(&wcnt[0][0])[tid + q * kBlockNT] = 0;
+    __syncthreads();
+    uint32_t pos[IPT];
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      if (static_cast<uint32_t>(j) < ipt) {
+        const bool valid = row0 + j * kWave < n;
+        const uint32_t d = digit_of(k[j], shift, dmask);
+        const uint64_t m = ballot(valid) & same_digit<8>(d);
+        const uint32_t below = mbcnt(m);
+        uint32_t prior = 0;
+        if (valid) {
+          prior = wcnt[w][d];
+          const uint32_t cnt = __popcll(m);
+          if (below == cnt - 1) wcnt[w][d] = static_cast<uint16_t>(prior + cnt);
+        }
+        pos[j] = prior + below;
+      }
+    }
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < kBins) {
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) total += wcnt[ww][tid];
+    }
+    uint32_t start = wave_incl_scan(total);
+    if (w < NBW && lane == kWave - 1) s_scan[w] = start;
+    start -= total;
+    __syncthreads();
+    if (tid < kBins) {
+#pragma unroll
+      for (int i = 0; i < NBW; ++i) start += static_cast<uint32_t>(i) < w ? s_scan[i] : 0u;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        const uint32_t c = wcnt[ww][tid];
+        wcnt[ww][tid] = static_cast<uint16_t>(start);
+        start += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      if (static_cast<uint32_t>(j) < ipt && row0 + j * kWave < n) {
+        const uint32_t at = pos[j] + wcnt[w][digit_of(k[j], shift, dmask)];
+        kbuf[at] = k[j];
+        if constexpr (VB > 0) vbuf[at] = v[j];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      const uint32_t i = row0 + j * kWave;
+      if (static_cast<uint32_t>(j) < ipt && i < n) {
+        k[j] = kbuf[i];
+        if constexpr (VB > 0) v[j] = vbuf[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const uint32_t i = row0 + j * kWave;
+    if (static_cast<uint32_t>(j) < ipt && i < n) {
+      keys[i] = k[j];
+      if constexpr (VB > 0) vals[i] = v[j];
+    }
+  }
+}
+
 template <int KB, int VB, int NT, int IPT, int DB, int LBW, class S>
 __global__ __launch_bounds__(NT, 4) void k_onesweep(
     typename Elem<KB>::T* __restrict__ k0, typename Elem<KB>::T* __restrict__ k1,
@@ -470,24 +620,7 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
       const uint64_t idx = wave_base + static_cast<uint64_t>(j) * kWave + lane;
       const bool valid = FULL || idx < n;
       const uint32_t d = dig<DB>(keys[j], shift, dmask);
-      // acc collects, per lane, the lanes whose digit differs in some bit:
-      // x is the lane's bit b as 0 or all ones, and acc | (bb ^ x) is one
-      // bitop3 per 32-bit half (table 0xDE with acc in the middle operand
-      // is the same under either operand order of the truth table).  Bits
-      // above a narrow last digit are zero everywhere and change nothing.
-      uint32_t acc_lo = 0, acc_hi = 0;
-#pragma unroll
-      for (int b = 0; b < DB; ++b) {
-        const uint32_t x = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(d), b, 1));
-        // The ballot of x itself (a plain ballot(x != 0) is rewritten into
-        // a second shift-and-compare of d); 33 is the not-equal predicate.
-        // Lanes outside exec give 0, as a ballot does.
-        const uint64_t bb = __builtin_amdgcn_uicmp(x, 0u, 33);
-        acc_lo = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(bb), acc_lo, x, 0xDE);
-        acc_hi = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(bb >> 32), acc_hi, x, 0xDE);
-      }
-      const uint64_t m =
-          (FULL ? ~0ull : ballot(valid)) & ~((static_cast<uint64_t>(acc_hi) << 32) | acc_lo);
+      const uint64_t m = (FULL ? ~0ull : ballot(valid)) & same_digit<DB>(d);
       const uint32_t below = mbcnt(m);
       const uint32_t cnt = __popcll(m);
       uint32_t prior = 0;
@@ -826,6 +959,16 @@ int sort_tuned(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
   if (n > kCountMask || ctx->tune_sort_status == 64)
     return sort_impl<KB, VB, Tn::NT, Tn::IPT, 8, kWindow, uint64_t>(ctx, keys, vals, n,
                                                                          key_bits);
+  if (n <= static_cast<uint64_t>(kBlockNT) * kBlockIPT<KB, VB> && !ctx->tune_sort_ipt &&
+      !ctx->tune_sort_digit) {
+    if (n < 2) return RFX_OK;
+    RFX_PROF(ctx, "sort.block");
+    k_sort_block<KB, VB><<<1, kBlockNT, 0, ctx->stream>>>(
+        static_cast<typename Elem<KB>::T*>(keys), static_cast<typename Elem<VB>::T*>(vals),
+        static_cast<uint32_t>(n), static_cast<uint32_t>(key_bits));
+    RFX_LAUNCHED();
+    return RFX_OK;
+  }
   if constexpr (kSortTunable<KB, VB>) {
     // Knob value 0 takes the digit width chosen for key_bits.
     const int digit = ctx->tune_sort_digit ? ctx->tune_sort_digit : auto_digit(key_bits);

@@ -247,3 +247,21 @@ def test_tile_queues_and_small_tiles_match_numpy(rf, ctx, kb, vb, bits, n):
     assert np.array_equal(gk, keys[order])
     if vb:
         assert np.array_equal(gv, vals[order])
+
+
+# Sorts of one block: steps and waves that are full, one row past, and the
+# last size (8192 rows, 4096 of 16-byte elements) with the next one; digits
+# that no key varies in, a narrow last digit, few distinct keys.
+@pytest.mark.parametrize("n", [2, 63, 65, 1024, 1025, 4096, 4097, 8191, 8192, 8193])
+@pytest.mark.parametrize("kb,vb,bits", [(4, 4, 32), (8, 4, 64), (8, 8, 61), (2, 1, 11), (1, 16, 8),
+                                        (16, 0, 128), (16, 16, 67), (4, 0, 5)])
+def test_one_block_sorts_match_oracle(rf, ctx, orc, kb, vb, bits, n):
+    keys = make(kb, n, 1100 + bits)
+    if kb >= 4:
+        keys.view(np.uint8)[kb - 2::kb] = 7  # a byte that is the same in every key
+    vals = make(vb, n, 1101) if vb else None
+    gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
+    ok, ov = orc.sort_pairs(keys, vals, kb, bits, vb)
+    assert np.array_equal(gk, ok)
+    if vb:
+        assert np.array_equal(gv, ov)
