@@ -3,12 +3,13 @@
 //
 // Keys are device addresses of NUL-terminated strings, each side sorted by
 // compare_string2 (ModernGPUJoin.cu:72-97): bytes compared as signed char
-// up to the first NUL of either, a proper prefix ordered first.  One
-// thread per left key finds the first right key not below it and the first
-// right key above it by binary search (every probe a string comparison in
-// global memory); the counts are then turned into their exclusive prefix
-// sums by a tile scan with decoupled look-back, whose last tile writes the
-// total.  The outputs are those of rfx_join_find_bounds, so rfx_join_main
+// up to the first NUL of either, a proper prefix ordered first.  A block of
+// left keys first narrows the right side to the range that its first and
+// last key span; one thread per left key then finds its lower bound in that
+// range (every probe a string comparison in global memory) and takes its
+// upper bound from its neighbour's lower bound; the counts are turned into
+// their exclusive prefix sums by a tile scan with decoupled look-back, whose
+// last tile writes the total.  The outputs are those of rfx_join_find_bounds, so rfx_join_main
 // expands them into row pairs.
 #include "rfx_device.h"
 #include "rfx_internal.h"
@@ -57,27 +58,89 @@ __device__ __forceinline__ bool str_less(uint64_t pa, uint64_t pb) {
 
 constexpr int kSNT = 256;
 
+// First index in [lo, hi) whose string is not below key (UPPER: above key),
+// by one wave: 64 probes a round, of which the ones below form a prefix.
+template <bool UPPER>
+__device__ __forceinline__ uint64_t wave_bound(const uint64_t* __restrict__ right, uint64_t lo,
+                                               uint64_t hi, uint64_t key) {
+  const uint32_t lane = lane_id();
+  while (lo < hi) {
+    const uint64_t len = hi - lo;
+    // Probe points, spread evenly; the same point may be taken twice.
+    const uint64_t at = lo + len * (lane + 1) / (kWave + 1);
+    const bool below = UPPER ? !str_less(key, right[at]) : str_less(right[at], key);
+    const uint32_t c = static_cast<uint32_t>(__popcll(ballot(below)));
+    const uint64_t old = lo;
+    if (c) lo = old + len * c / (kWave + 1) + 1;
+    if (c < kWave) hi = old + len * (c + 1) / (kWave + 1);
+  }
+  return lo;
+}
+
+// Searches are chains of dependent loads, so what counts is their length: at
+// 2^18 left and 2^22 right keys a search of all right keys is 22 probes and
+// the upper bound as many again.  The block's range costs 4 rounds of 64
+// probes for its first and last key (one wave each); inside it a thread
+// probes three points a round; the upper bound is the next key's lower
+// bound, which one comparison confirms (a right key that no left key equals
+// may lie in between: then the run is galloped over).
 __global__ __launch_bounds__(kSNT) void k_str_bounds(const uint64_t* __restrict__ left, uint64_t nl,
                                                      const uint64_t* __restrict__ right,
                                                      uint64_t nr, int32_t* __restrict__ lower,
                                                      int32_t* __restrict__ count) {
-  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kSNT + threadIdx.x;
-  if (i >= nl) return;
-  const uint64_t key = left[i];
-  uint64_t lo = 0, hi = nr;  // first right key not below key
-  while (lo < hi) {
-    const uint64_t mid = (lo + hi) >> 1;
-    if (str_less(right[mid], key)) lo = mid + 1;
-    else hi = mid;
+  __shared__ uint64_t s_range[2];
+  __shared__ uint64_t s_lo[kSNT];
+  const uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * kSNT;
+  const uint64_t i = i0 + threadIdx.x;
+  const uint64_t last = (i0 + kSNT < nl ? i0 + kSNT : nl) - 1;
+  const uint32_t w = wave_id();
+  if (w < 2) {
+    const uint64_t r = w == 0 ? wave_bound<false>(right, 0, nr, left[i0])
+                              : wave_bound<true>(right, 0, nr, left[last]);
+    if (lane_id() == 0) s_range[w] = r;
   }
-  uint64_t ub_lo = lo, ub_hi = nr;  // first right key above key
-  while (ub_lo < ub_hi) {
-    const uint64_t mid = (ub_lo + ub_hi) >> 1;
-    if (str_less(key, right[mid])) ub_hi = mid;
-    else ub_lo = mid + 1;
+  __syncthreads();
+  const uint64_t b0 = s_range[0], b1 = s_range[1];
+  const uint64_t key = i < nl ? left[i] : 0;
+  uint64_t lo = b0, hi = i < nl ? b1 : b0;  // first right key not below key
+  while (lo < hi) {
+    const uint64_t q = (hi - lo) / 4;
+    const uint64_t p0 = lo + q, p1 = lo + 2 * q, p2 = lo + 3 * q;
+    const uint64_t a0 = right[p0], a1 = right[p1], a2 = right[p2];
+    const bool l0 = str_less(a0, key), l1 = str_less(a1, key), l2 = str_less(a2, key);
+    hi = l2 ? hi : l1 ? p2 : l0 ? p1 : p0;
+    lo = l2 ? p2 + 1 : l1 ? p1 + 1 : l0 ? p0 + 1 : lo;
+  }
+  s_lo[threadIdx.x] = lo;
+  __syncthreads();
+  if (i >= nl) return;
+  // Every right key before `next` is not above the next left key's
+  // predecessor's range: the run of keys equal to this one ends there or
+  // before.
+  const uint64_t next = i == last ? b1 : s_lo[threadIdx.x + 1];
+  uint64_t up = lo;
+  if (next > lo && !str_less(key, right[next - 1])) {
+    up = next;
+  } else {
+    // Equal keys lie in [lo, end): gallop, then search.
+    uint64_t end = b1, step = 1;
+    while (up < b1) {
+      const uint64_t at = up + step - 1 < b1 ? up + step - 1 : b1 - 1;
+      if (str_less(key, right[at])) {
+        end = at;
+        break;
+      }
+      up = at + 1;
+      step <<= 1;
+    }
+    while (up < end) {
+      const uint64_t mid = (up + end) >> 1;
+      if (str_less(key, right[mid])) end = mid;
+      else up = mid + 1;
+    }
   }
   lower[i] = static_cast<int32_t>(lo);
-  count[i] = static_cast<int32_t>(ub_lo - lo);
+  count[i] = static_cast<int32_t>(up - lo);
 }
 
 // count[] -> exclusive prefix sums in place, tiles of 256 x 8; *total gets
@@ -130,48 +193,110 @@ __global__ __launch_bounds__(kSNT) void k_count_scan(int32_t* __restrict__ count
   if (tile == ntiles - 1 && tid == 0) *total = s_prefix + tile_sum;
 }
 
-// The order-preserving code of one byte of a string: the terminator 0,
-// then signed chars -128..-1, 1..127 as 1..255 (compare_string2's order).
-__device__ __forceinline__ uint64_t str_code(uint8_t b) {
-  return b == 0 ? 0u : static_cast<uint64_t>((b ^ 0x80u) + (b >= 0x80u ? 1u : 0u));
+// 8 bytes of a string as 8 order-preserving codes, first byte most
+// significant: the terminator and what follows it 0, then signed chars
+// -128..-1, 1..127 as 1..255 (compare_string2's order).
+__device__ __forceinline__ uint64_t str_codes(uint64_t v) {
+  const uint64_t z = zero_bytes(v);
+  if (z) v &= (1ull << (static_cast<uint32_t>(__builtin_ctzll(z)) & ~7u)) - 1;
+  const uint64_t some = (nonzero_bytes(v) >> 7) * 0xFFull;
+  // No carry leaves a byte: 0xFF becomes 0x7F + 1.
+  const uint64_t c = ((v ^ 0x8080808080808080ull) + ((v >> 7) & 0x0101010101010101ull)) & some;
+  return __builtin_bswap64(c);
 }
 
-// The longest string (bytes before the NUL; null addresses are empty)
-// into *longest, which starts at 0.
-__global__ __launch_bounds__(kSNT) void k_str_len(const uint64_t* __restrict__ addr, uint64_t n,
-                                                  uint64_t* __restrict__ longest) {
-  const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kSNT + threadIdx.x;
-  uint64_t k = 0;
-  if (i < n) {
-    const uint8_t* s = reinterpret_cast<const uint8_t*>(addr[i]);
-    if (s)
-      while (s[k]) ++k;
+// Walks a string 8 bytes at a time: the codes of the next 8 bytes, 0 past
+// the end.
+struct StrWalk {
+  uint64_t p;  // 0: ended
+  __device__ __forceinline__ explicit StrWalk(uint64_t addr) : p(addr) {}
+  __device__ __forceinline__ uint64_t next() {
+    if (!p) return 0;
+    const uint64_t v = load8(p);
+    p = zero_bytes(v) ? 0 : p + 8;
+    return str_codes(v);
   }
-  // One atomic per wave.
-  for (int d = kWave / 2; d > 0; d >>= 1) {
-    const uint64_t o = __shfl_xor(k, d, kWave);
-    k = o > k ? o : k;
-  }
-  if (lane_id() == 0 && k) atomicMax(reinterpret_cast<unsigned long long*>(longest), k);
+};
+
+// The bits of the strings' codes in which any string differs from the first
+// one, for the first kVaryWords words of 8 codes, and the number of words of
+// the longest string.
+constexpr int kVaryWords = 32;
+struct StrStats {
+  unsigned long long vary[kVaryWords];
+  unsigned long long words;
+};
+
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+  int x = static_cast<int>(v);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x |= __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(x, kWave - 1));
 }
 
-// Chunk c of every string as a big-endian key of 8 codes (codes past the
-// end are 0).  With rows, element i is the string of row rows[i].
-__global__ __launch_bounds__(kSNT) void k_str_chunk(const uint64_t* __restrict__ addr,
-                                                    const uint32_t* __restrict__ rows, uint64_t n,
-                                                    uint64_t chunk, uint64_t* __restrict__ key) {
+__global__ __launch_bounds__(kSNT) void k_str_stats(const uint64_t* __restrict__ addr, uint64_t n,
+                                                    StrStats* __restrict__ out) {
+  __shared__ unsigned long long s_vary[kVaryWords];
+  __shared__ uint32_t s_words;
+  for (uint32_t q = threadIdx.x; q < kVaryWords; q += kSNT) s_vary[q] = 0;
+  if (threadIdx.x == 0) s_words = 0;
+  __syncthreads();
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kSNT;
+  const uint64_t first = addr[0];
+  // Whole waves go round together; the last rows are repeated.
+  for (uint64_t i0 = static_cast<uint64_t>(blockIdx.x) * kSNT; i0 < n; i0 += stride) {
+    const uint64_t i = i0 + threadIdx.x < n ? i0 + threadIdx.x : n - 1;
+    StrWalk me(addr[i]), ref(first);
+    uint32_t c = 0;
+    while (ballot(me.p != 0 || ref.p != 0)) {
+      const uint64_t d = me.next() ^ ref.next();
+      if (c < kVaryWords) {
+        const uint64_t any = static_cast<uint64_t>(wave_or(static_cast<uint32_t>(d >> 32))) << 32 |
+                             wave_or(static_cast<uint32_t>(d));
+        if (lane_id() == 0 && any) atomicOr(&s_vary[c], any);
+      }
+      ++c;
+    }
+    if (lane_id() == 0) atomicMax(&s_words, c);
+  }
+  __syncthreads();
+  for (uint32_t q = threadIdx.x; q < kVaryWords; q += kSNT)
+    if (s_vary[q]) atomicOr(&out->vary[q], s_vary[q]);
+  if (threadIdx.x == 0 && s_words)
+    atomicMax(&out->words, static_cast<unsigned long long>(s_words));
+}
+
+// A sort key of up to 64 bits: pieces of the strings' code words, most
+// significant first.
+struct StrPiece {
+  uint32_t word;
+  uint8_t shift, bits;
+};
+struct StrKey {
+  int pieces;
+  StrPiece p[64];
+};
+
+// Each string's key.  With rows, element i is the string of row rows[i].
+template <class K>
+__global__ __launch_bounds__(kSNT) void k_str_key(const uint64_t* __restrict__ addr,
+                                                  const uint32_t* __restrict__ rows, uint64_t n,
+                                                  StrKey key, K* __restrict__ out) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * kSNT + threadIdx.x;
   if (i >= n) return;
-  const uint8_t* s = reinterpret_cast<const uint8_t*>(addr[rows ? rows[i] : i]);
-  uint64_t k = 0;
-  bool ended = s == nullptr;
-  for (uint64_t q = 0; q < 8 * chunk && !ended; ++q) ended = s[q] == 0;
-  for (int b = 0; b < 8; ++b) {
-    const uint8_t c = ended ? 0 : s[8 * chunk + b];
-    ended = ended || c == 0;
-    k = (k << 8) | str_code(c);
+  StrWalk s(addr[rows ? rows[i] : i]);
+  uint64_t k = 0, codes = s.next();
+  uint32_t at = 0;
+  for (int q = 0; q < key.pieces; ++q) {
+    const StrPiece p = key.p[q];
+    for (; at < p.word; ++at) codes = s.next();
+    k = p.bits < 64 ? (k << p.bits) | ((codes >> p.shift) & ((1ull << p.bits) - 1)) : codes;
   }
-  key[i] = k;
+  out[i] = static_cast<K>(k);
 }
 
 // Run heads of sorted strings: 1 where a string differs from the one
@@ -226,27 +351,83 @@ extern "C" int rfx_string_groups(rfx_ctx* ctx, const uint64_t* sorted, uint64_t 
   return RFX_OK;
 }
 
+namespace rfx {
+namespace {
+
+// Sort rows (or, without rows, the addresses themselves) by their strings.
+// Of each of the first kVaryWords words only the bits that differ between
+// strings go into the sort keys (in each code from its lowest to its highest
+// such bit), so names like Supplier#000012345 sort by one key of 4 bits a
+// varying digit instead of three 64-bit keys; later words go in whole.  LSD
+// over keys of up to 64 bits, least significant key first; each pass is a
+// stable sort of (key, payload) pairs.
+int sort_by_string(rfx_ctx* ctx, const uint64_t* addr, uint64_t* moved, uint32_t* rows,
+                   uint64_t* scratch, uint64_t n) {
+  RFX_TRY(ensure_workspace(ctx, sizeof(StrStats)));
+  StrStats* stats = static_cast<StrStats*>(ctx->ws);
+  RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(stats), sizeof(StrStats) / 4, 0));
+  const uint64_t blocks = (n + kSNT - 1) / kSNT, most = static_cast<uint64_t>(ctx->device_cus) * 16;
+  k_str_stats<<<static_cast<uint32_t>(blocks < most ? blocks : most), kSNT, 0, ctx->stream>>>(
+      addr, n, stats);
+  RFX_LAUNCHED();
+  StrStats h;
+  RFX_HIP(hipMemcpyAsync(&h, stats, sizeof h, hipMemcpyDeviceToHost, ctx->stream));
+  RFX_HIP(hipStreamSynchronize(ctx->stream));
+  // Pieces from the least significant end, cut into keys of up to 64 bits.
+  StrKey key{};
+  uint32_t bits = 0;
+  auto flush = [&]() -> int {
+    if (!bits) return RFX_OK;
+    for (int a = 0, b = key.pieces - 1; a < b; ++a, --b) {
+      const StrPiece t = key.p[a];
+      key.p[a] = key.p[b];
+      key.p[b] = t;
+    }
+    const int kb = bits <= 32 ? 4 : 8;
+    if (kb == 4)
+      k_str_key<uint32_t><<<static_cast<uint32_t>(blocks), kSNT, 0, ctx->stream>>>(
+          addr, rows, n, key, reinterpret_cast<uint32_t*>(scratch));
+    else
+      k_str_key<uint64_t><<<static_cast<uint32_t>(blocks), kSNT, 0, ctx->stream>>>(addr, rows, n,
+                                                                                   key, scratch);
+    RFX_LAUNCHED();
+    RFX_TRY(rfx_sort_pairs(ctx, scratch, rows ? static_cast<void*>(rows) : moved, n, kb,
+                           static_cast<int>(bits), rows ? 4 : 8));
+    key.pieces = 0;
+    bits = 0;
+    return RFX_OK;
+  };
+  auto piece = [&](uint64_t word, uint32_t shift, uint32_t width) -> int {
+    if (bits + width > 64) RFX_TRY(flush());
+    key.p[key.pieces++] = {static_cast<uint32_t>(word), static_cast<uint8_t>(shift),
+                           static_cast<uint8_t>(width)};
+    bits += width;
+    return RFX_OK;
+  };
+  for (uint64_t c = h.words; c-- > 0;) {
+    if (c >= kVaryWords) {
+      RFX_TRY(piece(c, 0, 64));
+      continue;
+    }
+    for (uint32_t sh = 0; sh < 64; sh += 8) {
+      const uint32_t v = static_cast<uint32_t>(h.vary[c] >> sh) & 0xFFu;
+      if (!v) continue;
+      const uint32_t lo = static_cast<uint32_t>(__builtin_ctz(v));
+      RFX_TRY(piece(c, sh + lo, 32u - static_cast<uint32_t>(__builtin_clz(v)) - lo));
+    }
+  }
+  return flush();
+}
+
+}  // namespace
+}  // namespace rfx
+
 extern "C" int rfx_sort_strings(rfx_ctx* ctx, uint64_t* addresses, uint64_t* scratch, uint64_t n) {
   if (!ctx || (n && (!addresses || !scratch)))
     return fail(RFX_EINVAL, "rfx_sort_strings: null argument");
   if (n < 2) return RFX_OK;
   if (n >= (1ull << 40)) return fail(RFX_ERANGE, "rfx_sort_strings: too many strings");
-  const uint32_t grid = static_cast<uint32_t>((n + kSNT - 1) / kSNT);
-  // The longest string fixes the number of passes (scratch[n] holds it).
-  RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(scratch + n), 2, 0));
-  k_str_len<<<grid, kSNT, 0, ctx->stream>>>(addresses, n, scratch + n);
-  RFX_LAUNCHED();
-  uint64_t longest = 0;
-  RFX_HIP(hipMemcpyAsync(&longest, scratch + n, 8, hipMemcpyDeviceToHost, ctx->stream));
-  RFX_HIP(hipStreamSynchronize(ctx->stream));
-  // LSD over 8-byte chunks, last chunk first: each pass a stable sort of
-  // (chunk key, address) pairs.
-  for (uint64_t chunk = (longest + 7) / 8; chunk-- > 0;) {
-    k_str_chunk<<<grid, kSNT, 0, ctx->stream>>>(addresses, nullptr, n, chunk, scratch);
-    RFX_LAUNCHED();
-    RFX_TRY(rfx_sort_pairs(ctx, scratch, addresses, n, 8, 64, 8));
-  }
-  return RFX_OK;
+  return sort_by_string(ctx, addresses, addresses, nullptr, scratch, n);
 }
 
 extern "C" int rfx_sort_strings_rows(rfx_ctx* ctx, const uint64_t* addresses, uint32_t* rows,
@@ -255,21 +436,7 @@ extern "C" int rfx_sort_strings_rows(rfx_ctx* ctx, const uint64_t* addresses, ui
     return fail(RFX_EINVAL, "rfx_sort_strings_rows: null argument");
   if (n >= (1ull << 32)) return fail(RFX_ERANGE, "rfx_sort_strings_rows: too many rows");
   if (n < 2) return RFX_OK;
-  const uint32_t grid = static_cast<uint32_t>((n + kSNT - 1) / kSNT);
-  RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(scratch + n), 2, 0));
-  k_str_len<<<grid, kSNT, 0, ctx->stream>>>(addresses, n, scratch + n);
-  RFX_LAUNCHED();
-  uint64_t longest = 0;
-  RFX_HIP(hipMemcpyAsync(&longest, scratch + n, 8, hipMemcpyDeviceToHost, ctx->stream));
-  RFX_HIP(hipStreamSynchronize(ctx->stream));
-  // As rfx_sort_strings, carrying row numbers: each pass keys the rows in
-  // their current order by the chunk of their own string.
-  for (uint64_t chunk = (longest + 7) / 8; chunk-- > 0;) {
-    k_str_chunk<<<grid, kSNT, 0, ctx->stream>>>(addresses, rows, n, chunk, scratch);
-    RFX_LAUNCHED();
-    RFX_TRY(rfx_sort_pairs(ctx, scratch, rows, n, 8, 64, 4));
-  }
-  return RFX_OK;
+  return sort_by_string(ctx, addresses, nullptr, rows, scratch, n);
 }
 
 extern "C" int rfx_join_find_bounds_string(rfx_ctx* ctx, int32_t* lower_bound, int32_t* left_count,

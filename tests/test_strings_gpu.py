@@ -269,3 +269,54 @@ def test_plan_like_tests(rf, ctx):
     assert p.get("L")[0].tolist() == [v for c, v in rows if oracle.like(c, b"%special%requests%")]
     assert p.get("N")[0].tolist() == [v for c, v in rows
                                       if not oracle.like(c, b"%requests%") and v < 500_000]
+
+
+# What goes into the sort keys: nothing (equal strings), one key of 4 or 8
+# bytes, several keys, whole words past the first 256 bytes; ends inside and
+# at the end of a word.
+@pytest.mark.parametrize("kind", ["equal", "digits", "wide", "long", "ends"])
+@pytest.mark.parametrize("rows", [False, True])
+def test_sort_strings_keys(rf, ctx, kind, rows):
+    rng = np.random.default_rng(5)
+    n = 9001
+    num = rng.integers(0, 3000, n)
+    if kind == "equal":
+        strings = [b"the same name"] * n
+    elif kind == "digits":
+        strings = [b"Supplier#%09d" % i for i in num]
+    elif kind == "wide":
+        strings = [bytes(rng.integers(1, 256, 11).astype(np.uint8)) + b"%03d" % (i % 7) for i in num]
+    elif kind == "long":
+        strings = [b"x" * (250 + int(i) % 20) + b"%04d" % i for i in num]
+    else:
+        strings = [b"\x01\xff\x7f\x80abcdefghijkl"[:int(i) % 17] for i in num]
+    buf, addr = strings_on_device(rf, strings)
+    scratch = rf.DeviceBuffer(8 * (n + 1))
+    before = addr.download(np.uint64, n)
+    order = sorted(range(n), key=lambda i: oracle.string_key(strings[i]))  # stable
+    if rows:
+        perm = rf.DeviceBuffer(4 * n)
+        ctx.iota_u32(perm, n)
+        ctx.sort_strings_rows(addr, perm, scratch, n)
+        assert perm.download(np.uint32, n).tolist() == order
+        assert np.array_equal(addr.download(np.uint64, n), before)
+    else:
+        ctx.sort_strings(addr, scratch, n)
+        assert np.array_equal(addr.download(np.uint64, n), before[order])
+
+
+# A block of left keys and its edges; runs of one left key over a whole
+# block; right keys between, before and after the left ones; nothing equal.
+@pytest.mark.parametrize("nl,nr,step,lstep", [(256, 5000, 1, 1), (257, 70_000, 3, 7), (513, 64, 2, 1),
+                                              (700, 4097, 1, 0), (1000, 3000, 0, 1), (5, 9000, 1, 900)])
+def test_find_bounds_string_ranges(rf, ctx, nl, nr, step, lstep):
+    left = [b"key%07d" % (100 + lstep * i) for i in range(nl)]
+    right = sorted(b"key%07d" % (step * (i // 3)) for i in range(nr))
+    lb_buf, lkeys = strings_on_device(rf, left)
+    rb_buf, rkeys = strings_on_device(rf, right)
+    lb, lc, tot = rf.DeviceBuffer(4 * nl), rf.DeviceBuffer(4 * nl), rf.u64_cell()
+    ctx.join_find_bounds_string(lb, lc, tot, lkeys, nl, rkeys, nr)
+    want_lb, want_lc, want_total = oracle.find_bounds_string(left, right)
+    assert rf.read_u64(tot) == want_total
+    assert np.array_equal(lb.download(np.int32, nl), want_lb)
+    assert np.array_equal(lc.download(np.int32, nl), want_lc)
