@@ -158,3 +158,24 @@ def test_q1_full_size_properties(rf, ctx):
     q = cols[3][keep].astype(np.int64)
     for grp in range(6):
         assert got[grp, 0] == float(q[g == grp].sum())
+
+
+# The interval that a comparison becomes, at its ends: constants 0, the
+# field's largest and smallest, the sign bit, and constants wider than the
+# field; 1 to 64 bit fields, one across the words of a 16-byte tuple.
+@pytest.mark.parametrize("tb,shift,bits", [(1, 2, 3), (4, 0, 32), (4, 31, 1), (8, 20, 33), (8, 0, 64),
+                                           (16, 50, 40), (16, 0, 64), (16, 64, 32), (16, 63, 1)])
+@pytest.mark.parametrize("op", range(10))
+def test_select_interval_ends(rf, ctx, orc, tb, shift, bits, op):
+    n = 30_007
+    rng = np.random.default_rng(tb + bits)
+    rows = rng.integers(0, 256, n * tb, dtype=np.uint8)
+    ends = np.array([0, 0, 1, 127, 128, 255], dtype=np.uint8)
+    rows[: n * tb // 2] = ends[rng.integers(0, 6, n * tb // 2)]  # fields at and near their ends
+    rows = rows.view({1: np.uint8, 2: np.uint16, 4: np.uint32}.get(tb, np.uint64)).copy()
+    top = (1 << bits) - 1
+    for k in {0, 1, top >> 1, (top >> 1) + 1, top - 1, top, (top + 1) & (2**64 - 1),
+              (1 << 63) | 5, 2**64 - 1, 2**64 - 1 - (top >> 1)}:
+        got = gpu_select(rf, ctx, rows, tb, shift, bits, op, k & (2**64 - 1))
+        want = orc.select(rows, tb, shift, bits, op, k & (2**64 - 1))
+        assert np.array_equal(got, want), (op, hex(k))
