@@ -106,6 +106,50 @@ uint32_t grid_of(uint64_t n) {
   return static_cast<uint32_t>(b ? b : 1);
 }
 
+// Device copy: a block moves kCopyBlock bytes, all its loads in flight before
+// the first store, and runs of kCopyRun blocks are neighbours on one XCD
+// (blockIdx is dealt out to the XCDs in turn), so each XCD streams through
+// pages of its own (2 GiB 0.885 -> 0.760 ms, 1 GiB 0.418 -> 0.378; the same as
+// the runtime up to 128 MiB).
+constexpr int kCopyNT = 512;
+constexpr int kCopyVT = 8;
+constexpr uint64_t kCopyBlock = 16ull * kCopyNT * kCopyVT;
+constexpr uint64_t kCopyMin = 64ull << 20;
+constexpr uint32_t kCopyRun = 32;
+
+__global__ __launch_bounds__(kCopyNT) void k_copy(const uint4* __restrict__ src,
+                                                  uint4* __restrict__ dst, uint64_t bytes) {
+  const uint32_t group = 8 * kCopyRun;
+  const uint32_t g0 = blockIdx.x / group * group, r = blockIdx.x % group;
+  uint32_t b = blockIdx.x;
+  if (g0 + group <= gridDim.x) b = g0 + (r % 8) * kCopyRun + r / 8;
+  const uint64_t at = static_cast<uint64_t>(b) * (kCopyNT * kCopyVT) + threadIdx.x;
+  const uint64_t full = bytes / 16;
+  if (static_cast<uint64_t>(b + 1) * (kCopyNT * kCopyVT) <= full) {
+    uint4 v[kCopyVT];
+#pragma unroll
+    for (int j = 0; j < kCopyVT; ++j) v[j] = src[at + j * kCopyNT];
+#pragma unroll
+    for (int j = 0; j < kCopyVT; ++j) dst[at + j * kCopyNT] = v[j];
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < kCopyVT; ++j)
+    if (at + j * kCopyNT < full) dst[at + j * kCopyNT] = src[at + j * kCopyNT];
+  const uint64_t tail = full * 16 + threadIdx.x;  // the last bytes, by the last block
+  if (b == gridDim.x - 1 && tail < bytes)
+    reinterpret_cast<uint8_t*>(dst)[tail] = reinterpret_cast<const uint8_t*>(src)[tail];
+}
+
+bool own_memory(rfx_ctx* ctx, const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == ctx->device;
+}
+
 }  // namespace
 }  // namespace rfx
 
@@ -136,12 +180,14 @@ int rfx_graph_begin(rfx_ctx* ctx) {
   if (ctx->profiling) return fail(RFX_EINVAL, "rfx_graph_begin: disable profiling first");
   RFX_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   ctx->capturing = true;
+  ++g_capturing;
   return RFX_OK;
 }
 
 int rfx_graph_end(rfx_ctx* ctx, void** graph_exec) {
   if (!ctx || !graph_exec) return fail(RFX_EINVAL, "rfx_graph_end: null argument");
   hipGraph_t g = nullptr;
+  if (ctx->capturing) --g_capturing;
   ctx->capturing = false;
   RFX_HIP(hipStreamEndCapture(ctx->stream, &g));
   hipGraphExec_t e = nullptr;
@@ -180,7 +226,20 @@ int rfx_graph_destroy(void* graph_exec) {
 
 int rfx_copy(rfx_ctx* ctx, void* dst, const void* src, uint64_t bytes) {
   if (!ctx || (bytes && (!dst || !src))) return fail(RFX_EINVAL, "rfx_copy: null argument");
-  if (bytes) RFX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+  if (!bytes) return RFX_OK;
+  // A large copy between this device's own allocations; the runtime's copy
+  // takes any other pointers (and small copies, which are all launch).
+  if (bytes >= kCopyMin && reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(src) % 16 == 0 && own_memory(ctx, dst) && own_memory(ctx, src)) {
+    const uint64_t blocks = (bytes + kCopyBlock - 1) / kCopyBlock;
+    if (blocks <= 0x7FFFFFFFull) {
+      k_copy<<<static_cast<uint32_t>(blocks), kCopyNT, 0, ctx->stream>>>(
+          static_cast<const uint4*>(src), static_cast<uint4*>(dst), bytes);
+      RFX_LAUNCHED();
+      return RFX_OK;
+    }
+  }
+  RFX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
   return RFX_OK;
 }
 
