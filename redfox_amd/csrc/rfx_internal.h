@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -42,6 +43,9 @@ struct rfx_ctx {
 };
 
 namespace rfx {
+
+// Contexts between rfx_graph_begin and rfx_graph_end.
+extern std::atomic<int> g_capturing;
 
 // Record an error message for rfx_last_error() and return `code`.
 int fail(int code, const char* fmt, ...);

@@ -131,3 +131,37 @@ def test_q1_plan_from_lineitem_text(rf, ctx):
         sel = keep & (g == k)
         want = (price * (1 - disc) * (1 + tax))[sel].sum()
         assert abs(got - want) <= 1e-12 * abs(want)
+
+
+@pytest.mark.parametrize("size", [1 << 20, (64 << 20) + 5, (64 << 20) - 16, (66 << 20) + 65_536 * 3 + 16])
+def test_copies_of_any_size(rf, ctx, size):
+    """rfx_copy below and past the size where its own kernel takes over:
+    whole blocks, a last block, last bytes, and an unaligned source."""
+    src, dst = rf.DeviceBuffer(size + 16), rf.DeviceBuffer(size + 16)
+    ctx.gen_u32(src, (size + 16) // 4, 5)
+    want = src.download(np.uint8, size + 16)
+    for off in (0, 3):
+        dst.zero()
+        ctx.copy(dst, src, size, dst_off=0, src_off=off)
+        ctx.synchronize()
+        got = dst.download(np.uint8, size + 16)
+        assert np.array_equal(got[:size], want[off:size + off]) and not got[size:].any()
+
+
+def test_freed_blocks_are_handed_out_again_whole(rf):
+    """Blocks that rfx_free keeps: of the size asked for or more, never two
+    owners, whatever the order; sizes that are not kept."""
+    rng = np.random.default_rng(3)
+    live = []
+    for step in range(300):
+        if live and rng.random() < 0.5:
+            buf, tag = live.pop(int(rng.integers(len(live))))
+            assert (buf.download(np.uint8) == tag).all()
+            buf.close()
+        else:
+            n = int(rng.choice([1, 255, 4097, 100_000, 3 << 20, (64 << 20) + 1]) + rng.integers(0, 50))
+            buf = rf.DeviceBuffer(n)
+            assert rf.lib().rfx_memset(buf.ptr, step % 251, n) == 0
+            live.append((buf, step % 251))
+    for buf, tag in live:
+        assert (buf.download(np.uint8) == tag).all()
