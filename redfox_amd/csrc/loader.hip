@@ -30,44 +30,52 @@ constexpr int kLBytes = 64;
 constexpr int kLTile = kLNT * kLBytes;
 constexpr int kMaxFields = RFX_TBL_MAX_COLS;
 
+// Which of 4 bytes equal pat's (one byte four times): bits 0 to 3.
+__device__ __forceinline__ uint32_t byte_bits4(uint32_t w, uint32_t pat) {
+  const uint32_t x = w ^ pat;
+  // 0x80 in every zero byte (exact), moved together by one multiplication.
+  const uint32_t z = ~(((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x | 0x7F7F7F7Fu);
+  return ((z >> 7) * 0x10204080u) >> 28;
+}
+__device__ __forceinline__ uint32_t byte_bits16(uint4 v, uint32_t pat) {
+  return byte_bits4(v.x, pat) | byte_bits4(v.y, pat) << 4 | byte_bits4(v.z, pat) << 8 |
+         byte_bits4(v.w, pat) << 12;
+}
+
 __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ text,
                                                    uint64_t bytes, bool aligned,
                                                    uint64_t* __restrict__ ends,
                                                    uint64_t cap, uint32_t ntiles,
-                                                   uint64_t* __restrict__ n_newlines,
+                                                   uint64_t* __restrict__ counts,
+                                                   uint64_t* __restrict__ rows,
                                                    uint64_t* __restrict__ status,
                                                    uint32_t* __restrict__ ticket) {
   __shared__ uint32_t s_scan[kLNT / kWave + 1];
   __shared__ uint32_t s_tile;
   __shared__ uint64_t s_prefix;
+  __shared__ __attribute__((aligned(8))) uint16_t s_bits[kLTile / 16];
   const uint32_t tid = threadIdx.x, lane = lane_id(), w = wave_id();
   if (tid == 0) s_tile = atomicAdd(ticket, 1u);
   __syncthreads();
   const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);  // block-uniform: scalar from here
-  const uint64_t at = static_cast<uint64_t>(tile) * kLTile + static_cast<uint64_t>(tid) * kLBytes;
-  // The thread's 64 bytes as sixteen words; bytes past the end are not
-  // newlines.
-  uint32_t word[kLBytes / 4];
-  if (aligned && at + kLBytes <= bytes) {
+  const uint64_t tile_at = static_cast<uint64_t>(tile) * kLTile;
+  const uint64_t at = tile_at + static_cast<uint64_t>(tid) * kLBytes;
+  uint64_t mask = 0;  // bit b: byte b of the thread's 64 is a newline
+  if (aligned && tile_at + kLTile <= bytes) {  // uniform
+    // Neighbouring lanes load neighbouring 16 bytes; the newlines of each
+    // become 16 bits in LDS, where a thread then reads its 64 bytes' bits.
+    const uint4* t = reinterpret_cast<const uint4*>(text + tile_at) + tid;
+    uint4 v[kLBytes / 16];
 #pragma unroll
-    for (int j = 0; j < kLBytes / 16; ++j) {
-      const uint4 v = reinterpret_cast<const uint4*>(text + at)[j];
-      word[4 * j] = v.x;
-      word[4 * j + 1] = v.y;
-      word[4 * j + 2] = v.z;
-      word[4 * j + 3] = v.w;
-    }
+    for (int j = 0; j < kLBytes / 16; ++j) v[j] = t[j * kLNT];
+#pragma unroll
+    for (int j = 0; j < kLBytes / 16; ++j)
+      s_bits[tid + j * kLNT] = static_cast<uint16_t>(byte_bits16(v[j], 0x0A0A0A0Au));
+    __syncthreads();
+    mask = reinterpret_cast<const uint64_t*>(s_bits)[tid];
   } else {
-#pragma unroll
-    for (int j = 0; j < kLBytes / 4; ++j) word[j] = 0;
     for (int b = 0; b < kLBytes; ++b)
-      if (at + b < bytes) word[b >> 2] |= static_cast<uint32_t>(text[at + b]) << (8 * (b & 3));
-  }
-  uint64_t mask = 0;  // bit b: byte b is a newline
-#pragma unroll
-  for (int b = 0; b < kLBytes; ++b) {
-    const uint32_t c = (word[b >> 2] >> (8 * (b & 3))) & 0xFF;
-    mask |= static_cast<uint64_t>(c == '\n' && at + b < bytes) << b;
+      if (at + b < bytes && text[at + b] == '\n') mask |= 1ull << b;
   }
   uint32_t total = 0;
   const uint32_t excl = block_excl_scan<kLNT>(static_cast<uint32_t>(__popcll(mask)), s_scan, &total);
@@ -94,7 +102,14 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
     if (k < cap) ends[k] = at + b;
     ++k;
   }
-  if (tile == ntiles - 1 && tid == 0) *n_newlines = s_prefix + total;
+  if (tile == ntiles - 1 && tid == 0) {
+    // The text's rows: a last one may end without a newline.
+    const uint64_t newlines = s_prefix + total;
+    const uint64_t n = newlines + (text[bytes - 1] != '\n' ? 1 : 0);
+    counts[0] = newlines;
+    counts[1] = n;
+    *rows = n;
+  }
 }
 
 struct TblCols {
@@ -301,36 +316,30 @@ extern "C" int rfx_tbl_parse(rfx_ctx* ctx, void* text, uint64_t bytes, char deli
   c.take<uint64_t>(ecap);
   c.take<uint64_t>(ntiles ? ntiles : 1);
   c.take<uint32_t>(1);
-  c.take<uint64_t>(1);
+  c.take<uint64_t>(2);
   RFX_TRY(ensure_workspace(ctx, c.off));
   Carve w(ctx->ws);
   uint64_t* ends = w.take<uint64_t>(ecap);
   uint64_t* status = w.take<uint64_t>(ntiles ? ntiles : 1);
   uint32_t* ticket = w.take<uint32_t>(1);
-  uint64_t* n_nl = w.take<uint64_t>(1);
+  uint64_t* counts = w.take<uint64_t>(2);  // newlines, rows
   RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(status),
-                   (reinterpret_cast<char*>(n_nl + 1) - reinterpret_cast<char*>(status)) / 4, 0));
+                   (reinterpret_cast<char*>(counts + 2) - reinterpret_cast<char*>(status)) / 4, 0));
   RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(short_rows), 2, 0));
-  uint64_t newlines = 0;
+  if (!ntiles) RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(rows), 2, 0));
   if (ntiles) {
     RFX_PROF(ctx, "tbl.rows");
     k_tbl_rows<<<static_cast<uint32_t>(ntiles), kLNT, 0, ctx->stream>>>(
         static_cast<const uint8_t*>(text), bytes, reinterpret_cast<uintptr_t>(text) % 16 == 0, ends,
-        ecap, static_cast<uint32_t>(ntiles), n_nl, status, ticket);
+        ecap, static_cast<uint32_t>(ntiles), counts, rows, status, ticket);
     RFX_LAUNCHED();
   }
   // The row count sizes the field pass: read it back.
-  RFX_HIP(hipMemcpyAsync(&newlines, n_nl, 8, hipMemcpyDeviceToHost, ctx->stream));
+  uint64_t got[2] = {0, 0};
+  if (ntiles && capacity && n_fields)
+    RFX_HIP(hipMemcpyAsync(got, counts, 16, hipMemcpyDeviceToHost, ctx->stream));
   RFX_HIP(hipStreamSynchronize(ctx->stream));
-  if (!ntiles) newlines = 0;
-  uint8_t last = 0;
-  if (bytes) {
-    RFX_HIP(hipMemcpyAsync(&last, static_cast<const uint8_t*>(text) + bytes - 1, 1,
-                           hipMemcpyDeviceToHost, ctx->stream));
-    RFX_HIP(hipStreamSynchronize(ctx->stream));
-  }
-  const uint64_t n = newlines + (bytes && last != '\n' ? 1 : 0);
-  RFX_HIP(hipMemcpyAsync(rows, &n, 8, hipMemcpyHostToDevice, ctx->stream));
+  const uint64_t newlines = got[0], n = got[1];
   const uint64_t todo = n < capacity ? n : capacity;
   if (todo && n_fields) {
     RFX_PROF(ctx, "tbl.fields");
@@ -338,7 +347,7 @@ extern "C" int rfx_tbl_parse(rfx_ctx* ctx, void* text, uint64_t bytes, char deli
         static_cast<uint8_t*>(text), bytes, reinterpret_cast<uintptr_t>(text) % 16 == 0,
         ends, newlines, todo, static_cast<uint8_t>(delim), n_fields, cols, short_rows);
     RFX_LAUNCHED();
+    RFX_HIP(hipStreamSynchronize(ctx->stream));
   }
-  RFX_HIP(hipStreamSynchronize(ctx->stream));
   return RFX_OK;
 }
