@@ -3,14 +3,13 @@
 // getline, strtok on the delimiter, atoi per field, one packed tuple per
 // row) as two HBM passes over the text once it is resident:
 //
-//  1. row ends: tiles of 512 threads x 64 bytes count the newlines in each
-//     thread's 64 bytes, scan the counts across the block and take the
-//     tile's offset from a decoupled look-back, then store the position of
-//     every newline in text order;
-//  2. fields: a block of 256 rows stages their text (one contiguous span)
-//     in LDS with 16-byte loads; one thread per row then walks its bytes,
-//     splitting at the delimiter, and converts field f by the type spec[f]
-//     straight into column f.
+//  1. row ends: tiles of 512 threads x 256 bytes turn the newlines into
+//     bits, count them, scan the counts across the block and take the tile's
+//     offset from a decoupled look-back, then store the position of every
+//     newline in text order;
+//  2. fields: a block of 128 rows stages their text (one contiguous span)
+//     in LDS; a thread per row splits it at the delimiters; then each wave
+//     converts field f of 64 rows by the type spec[f] into column f.
 //
 // Field conversions (C semantics): integers as atoi/atol (leading spaces,
 // a sign, digits up to the first other byte; wrapping), decimals as the
@@ -26,7 +25,11 @@ namespace rfx {
 namespace {
 
 constexpr int kLNT = 512;
-constexpr int kLBytes = 64;
+// Bytes per thread: 64 KB tiles.  Tiles take turns at one ticket word (12 ns
+// each) and at the look-back, so small tiles wait for those, large ones
+// leave the chip half empty: 133 MB of text in 16 KB tiles 118 us, 32 KB 72,
+// 64 KB 67, 128 KB 86.
+constexpr int kLBytes = 128;
 constexpr int kLTile = kLNT * kLBytes;
 constexpr int kMaxFields = RFX_TBL_MAX_COLS;
 
@@ -60,10 +63,10 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
   const uint32_t tile = __builtin_amdgcn_readfirstlane(s_tile);  // block-uniform: scalar from here
   const uint64_t tile_at = static_cast<uint64_t>(tile) * kLTile;
   const uint64_t at = tile_at + static_cast<uint64_t>(tid) * kLBytes;
-  uint64_t mask = 0;  // bit b: byte b of the thread's 64 is a newline
+  uint64_t mask[kLBytes / 64];  // bit b of word q: byte 64 q + b is a newline
   if (aligned && tile_at + kLTile <= bytes) {  // uniform
     // Neighbouring lanes load neighbouring 16 bytes; the newlines of each
-    // become 16 bits in LDS, where a thread then reads its 64 bytes' bits.
+    // become 16 bits in LDS, where a thread then reads its own bytes' bits.
     const uint4* t = reinterpret_cast<const uint4*>(text + tile_at) + tid;
     uint4 v[kLBytes / 16];
 #pragma unroll
@@ -72,13 +75,22 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
     for (int j = 0; j < kLBytes / 16; ++j)
       s_bits[tid + j * kLNT] = static_cast<uint16_t>(byte_bits16(v[j], 0x0A0A0A0Au));
     __syncthreads();
-    mask = reinterpret_cast<const uint64_t*>(s_bits)[tid];
+#pragma unroll
+    for (int q = 0; q < kLBytes / 64; ++q)
+      mask[q] = reinterpret_cast<const uint64_t*>(s_bits)[tid * (kLBytes / 64) + q];
   } else {
-    for (int b = 0; b < kLBytes; ++b)
-      if (at + b < bytes && text[at + b] == '\n') mask |= 1ull << b;
+#pragma unroll
+    for (int q = 0; q < kLBytes / 64; ++q) {
+      mask[q] = 0;
+      for (int b = 0; b < 64; ++b)
+        if (at + 64 * q + b < bytes && text[at + 64 * q + b] == '\n') mask[q] |= 1ull << b;
+    }
   }
+  uint32_t mine = 0;
+#pragma unroll
+  for (int q = 0; q < kLBytes / 64; ++q) mine += static_cast<uint32_t>(__popcll(mask[q]));
   uint32_t total = 0;
-  const uint32_t excl = block_excl_scan<kLNT>(static_cast<uint32_t>(__popcll(mask)), s_scan, &total);
+  const uint32_t excl = block_excl_scan<kLNT>(mine, s_scan, &total);
   if (w == 0) {
     if (tile == 0) {
       if (lane == 0) {
@@ -96,11 +108,14 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
   }
   __syncthreads();
   uint64_t k = s_prefix + excl;
-  while (mask) {
-    const int b = __builtin_ctzll(mask);
-    mask &= mask - 1;
-    if (k < cap) ends[k] = at + b;
-    ++k;
+#pragma unroll
+  for (int q = 0; q < kLBytes / 64; ++q) {
+    while (mask[q]) {
+      const int b = __builtin_ctzll(mask[q]);
+      mask[q] &= mask[q] - 1;
+      if (k < cap) ends[k] = at + 64 * q + b;
+      ++k;
+    }
   }
   if (tile == ntiles - 1 && tid == 0) {
     // The text's rows: a last one may end without a newline.
@@ -109,6 +124,49 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
     counts[0] = newlines;
     counts[1] = n;
     *rows = n;
+  }
+}
+
+// The newlines alone, without their places: no order, so no ticket and no
+// look-back (133 MB: 29 us against 64 by the pass above).  counts[0] is 0
+// before; the last block to finish turns it into the rows.
+constexpr int kCNT = 512;
+__global__ __launch_bounds__(kCNT) void k_tbl_count(const uint8_t* __restrict__ text,
+                                                    uint64_t bytes, bool aligned,
+                                                    uint64_t* __restrict__ counts,
+                                                    uint64_t* __restrict__ rows,
+                                                    uint32_t* __restrict__ finished) {
+  __shared__ uint32_t s_sum[kCNT / kWave];
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kCNT;
+  const uint64_t g = static_cast<uint64_t>(blockIdx.x) * kCNT + threadIdx.x;
+  uint32_t mine = 0;
+  uint64_t done = 0;
+  if (aligned) {
+    const uint4* t = reinterpret_cast<const uint4*>(text);
+    const uint64_t vecs = bytes / 16;
+    uint64_t i = g;
+    for (; i + 3 * stride < vecs; i += 4 * stride) {
+      uint4 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = t[i + j * stride];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mine += __popc(byte_bits16(v[j], 0x0A0A0A0Au));
+    }
+    for (; i < vecs; i += stride) mine += __popc(byte_bits16(t[i], 0x0A0A0A0Au));
+    done = vecs * 16;
+  }
+  for (uint64_t i = done + g; i < bytes; i += stride) mine += text[i] == '\n';
+  const uint32_t w = wave_incl_scan(mine);
+  if (lane_id() == kWave - 1) s_sum[wave_id()] = w;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t sum = 0;
+    for (int i = 0; i < kCNT / kWave; ++i) sum += s_sum[i];
+    // The old value is waited for: the sum is in before the block is counted.
+    const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long*>(counts), sum);
+    asm volatile("" ::"v"(old) : "memory");
+    if (atomicAdd(finished, 1u) == gridDim.x - 1)
+      *rows = status_load64(counts) + (text[bytes - 1] != '\n' ? 1 : 0);
   }
 }
 
@@ -134,8 +192,9 @@ __device__ const double kPow10[23] = {1e0,  1e1,  1e2,  1e3,  1e4,  1e5,  1e6,  
                                       1e8,  1e9,  1e10, 1e11, 1e12, 1e13, 1e14, 1e15,
                                       1e16, 1e17, 1e18, 1e19, 1e20, 1e21, 1e22};
 
-constexpr int kFNT = 256;            // rows per block
-constexpr int kStage = 48 * 1024;     // staged text bytes per block
+constexpr int kFNT = 256;
+constexpr int kFRows = 128;           // rows per block
+constexpr int kStage = 24 * 1024;     // staged text bytes per block
 
 // Parse row r ([pos, end) of the text) into the columns; at(q) gives byte
 // q and scan(q, e) the first delimiter in [q, e) (e if none).  Each field's
@@ -214,75 +273,273 @@ __device__ __forceinline__ void parse_row(At at, Scan scan, uint8_t* text, uint6
   }
 }
 
-// Rows [256 b, 256 b + 256) of block b.  Their text is one contiguous span:
-// when it fits, the block stages it in LDS with 16-byte loads and every
-// thread parses its row from there; otherwise from global memory.
+// 8 bytes of the staged text from byte q (the stage ends in 16 spare bytes).
+__device__ __forceinline__ uint64_t lds8(const uint4* stage, uint32_t q) {
+  const uint64_t* w = reinterpret_cast<const uint64_t*>(stage) + (q >> 3);
+  const uint32_t sh = (q & 7) * 8;
+  const uint64_t lo = w[0], hi = w[1];
+  return lo >> sh | (hi << 1) << (63 - sh);
+}
+
+// The first n (1 to 8) bytes of w as decimal digits: value, and whether all
+// of them are digits.
+__device__ __forceinline__ bool digits8(uint64_t w, uint32_t n, uint32_t* value) {
+  const uint32_t pad = 8 * (8 - n);
+  const uint64_t x = (w ^ 0x3030303030303030ull) << pad;  // zeros first, then the digits
+  const uint64_t bad = (x | (x + 0x7676767676767676ull)) & 0x8080808080808080ull;
+  uint32_t four[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t y = static_cast<uint32_t>(x >> (32 * h));
+    const uint32_t two = (y & 0x00FF00FFu) * 10 + ((y >> 8) & 0x00FF00FFu);
+    four[h] = (two & 0xFFFFu) * 100 + (two >> 16);
+  }
+  *value = four[0] * 10000 + four[1];
+  return !bad;
+}
+
+// A field's bytes one at a time, from a register refilled every 8.
+struct FieldBytes {
+  const uint4* stage;
+  uint32_t q, e, left = 0;
+  uint64_t w = 0;
+  __device__ __forceinline__ bool more() const { return q < e; }
+  __device__ __forceinline__ uint8_t peek() {
+    if (!left) {
+      w = lds8(stage, q);
+      left = 8;
+    }
+    return static_cast<uint8_t>(w);
+  }
+  __device__ __forceinline__ void skip() {  // after peek
+    ++q;
+    w >>= 8;
+    --left;
+  }
+};
+
+// Staged field [s, e) as type t (uniform over the wave): the well-formed
+// ones by words, the others byte by byte, as parse_row reads them.
+__device__ __forceinline__ void parse_staged(const uint4* stage, uint32_t s, uint32_t e, int t,
+                                             int64_t* iv, double* dv) {
+  const uint32_t len = e - s;
+  if (t == RFX_TBL_CHAR) {
+    *iv = len ? reinterpret_cast<const uint8_t*>(stage)[s] : 0;
+    return;
+  }
+  const uint64_t w = lds8(stage, s);
+  if (t == RFX_TBL_DATE) {
+    uint32_t y, m, d;
+    const bool fine = len == 10 && static_cast<uint8_t>(w >> 32) == '-' &&
+                      static_cast<uint8_t>(w >> 56) == '-' && digits8(w, 4, &y) &&
+                      digits8(w >> 40, 2, &m) && digits8(lds8(stage, s + 8), 2, &d);
+    if (fine) {
+      *iv = static_cast<int64_t>(date2int(static_cast<int>(y), static_cast<int>(m),
+                                          static_cast<int>(d)));
+      return;
+    }
+    FieldBytes b{stage, s, e};
+    int part[3] = {0, 0, 0}, k = 0, state = 0;  // 0 leading, 1 digits, 2 done
+    for (; b.more() && k < 3; b.skip()) {
+      const uint8_t c = b.peek();
+      if (c == '-') {
+        ++k;
+        state = 0;
+      } else if (c >= '0' && c <= '9' && state < 2) {
+        const int digit = c - '0';
+        if (k == 0) part[0] = part[0] * 10 + digit;
+        else if (k == 1) part[1] = part[1] * 10 + digit;
+        else part[2] = part[2] * 10 + digit;
+        state = 1;
+      } else if (!(state == 0 && (c == ' ' || c == '+'))) {
+        state = 2;
+      }
+    }
+    *iv = static_cast<int64_t>(date2int(part[0], part[1], part[2]));
+    return;
+  }
+  uint32_t whole, part;
+  if (t == RFX_TBL_F64) {
+    // Up to 8 digits, or up to 7, a point and one or two more.
+    const uint64_t x = w ^ 0x2E2E2E2E2E2E2E2Eull;
+    const uint64_t z = (x - 0x0101010101010101ull) & ~x & 0x8080808080808080ull;
+    const uint32_t dot = z ? static_cast<uint32_t>(__builtin_ctzll(z)) >> 3 : 8;
+    const uint32_t after = len - dot - 1;  // digits after the point
+    if (dot >= len) {
+      if (len >= 1 && len <= 8 && digits8(w, len, &whole)) {
+        *dv = static_cast<double>(whole);
+        return;
+      }
+    } else if (dot >= 1 && dot < 8 && (after == 1 || after == 2) && digits8(w, dot, &whole) &&
+               digits8(lds8(stage, s + dot + 1), after, &part)) {
+      const uint32_t ten = after == 1 ? 10u : 100u;
+      *dv = static_cast<double>(whole * ten + part) / static_cast<double>(ten);
+      return;
+    }
+  } else if (len >= 1 && len <= 8 && digits8(w, len, &whole)) {
+    *iv = whole;
+    return;
+  }
+  FieldBytes b{stage, s, e};
+  while (b.more() && b.peek() == ' ') b.skip();
+  bool neg = false;
+  if (b.more() && (b.peek() == '-' || b.peek() == '+')) {
+    neg = b.peek() == '-';
+    b.skip();
+  }
+  uint64_t m = 0;
+  int frac = -1;  // digits after the point
+  for (; b.more(); b.skip()) {
+    const uint8_t c = b.peek();
+    if (c >= '0' && c <= '9') {
+      m = m * 10 + (c - '0');
+      if (frac >= 0) ++frac;
+    } else if (c == '.' && t == RFX_TBL_F64 && frac < 0) {
+      frac = 0;
+    } else {
+      break;
+    }
+  }
+  *iv = neg ? -static_cast<int64_t>(m) : static_cast<int64_t>(m);
+  if (t == RFX_TBL_F64) {
+    const double mag = static_cast<double>(m) / kPow10[frac > 0 ? (frac < 22 ? frac : 22) : 0];
+    *dv = neg ? -mag : mag;
+  }
+}
+
+// The fields that have a column, and how many fields a row is split into.
+struct TblTasks {
+  int n, fields;
+  uint8_t f[kMaxFields];
+};
+
+// Rows [128 b, 128 b + 128) of block b.  Their text is one contiguous span:
+// when it fits, the block stages it in LDS with 16-byte loads, one bit per
+// byte for the delimiters beside it; a thread per row walks those bits to
+// the ends of its fields; then each wave takes one field of 64 rows at a
+// time, so that its lanes convert texts of one type and their stores are
+// neighbours.  (A thread walking and converting a whole row was bound by its
+// chain of byte loads from LDS and by divergence, 12 waves per CU: 1 M
+// lineitem rows 144 us; now 99.)  Otherwise every thread parses a row
+// from global memory.
+constexpr uint16_t kNoField = 0xFFFF;  // past the fields that a row has
+
 __global__ __launch_bounds__(kFNT) void k_tbl_fields(uint8_t* __restrict__ text,
                                                      uint64_t bytes, bool aligned,
                                                      const uint64_t* __restrict__ ends,
                                                      uint64_t n_newlines, uint64_t rows,
-                                                     uint8_t delim, int n_fields, TblCols cols,
+                                                     uint8_t delim, TblTasks tasks, TblCols cols,
                                                      uint64_t* __restrict__ short_rows) {
-  __shared__ uint4 s_text[kStage / 16];
+  __shared__ uint4 s_text[kStage / 16 + 1];
+  __shared__ __attribute__((aligned(8))) uint16_t s_bits[kStage / 16 + 4];
+  __shared__ uint16_t s_start[kFRows];
   __shared__ uint64_t s_span[2];
-  const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kFNT;
-  if (threadIdx.x == 0) {
-    const uint64_t last = r0 + kFNT - 1 < rows ? r0 + kFNT - 1 : rows - 1;
+  extern __shared__ uint16_t s_ends[];  // [fields][kFRows]
+  const uint32_t tid = threadIdx.x;
+  const uint64_t r0 = static_cast<uint64_t>(blockIdx.x) * kFRows;
+  if (tid == 0) {
+    const uint64_t last = r0 + kFRows - 1 < rows ? r0 + kFRows - 1 : rows - 1;
     s_span[0] = r0 == 0 ? 0 : ends[r0 - 1] + 1;
     s_span[1] = last < n_newlines ? ends[last] : bytes;
   }
+  const uint64_t r = r0 + tid;
+  const bool mine = tid < kFRows && r < rows;
+  uint64_t pos = 0, end = 0;
+  if (mine) {
+    pos = r == 0 ? 0 : ends[r - 1] + 1;
+    end = r < n_newlines ? ends[r] : bytes;
+  }
   __syncthreads();
   const uint64_t base = s_span[0] & ~15ull, stop = s_span[1];
-  const bool staged = aligned && stop - base <= static_cast<uint64_t>(kStage);
-  if (staged) {
-    const uint32_t nvec = static_cast<uint32_t>((stop - base + 15) / 16);
-    for (uint32_t v = threadIdx.x; v < nvec; v += kFNT) {
-      const uint64_t off = base + 16ull * v;
+  if (!aligned || stop - base > static_cast<uint64_t>(kStage)) {
+    if (mine) {
+      auto scan = [&](uint64_t q, uint64_t e) -> uint64_t {
+        while (q < e && text[q] != delim) ++q;
+        return q;
+      };
+      parse_row([&](uint64_t q) -> uint8_t { return text[q]; }, scan, text, bytes, r, pos, end,
+                tasks.fields, cols, short_rows);
+    }
+    return;
+  }
+  constexpr int kVecs = kStage / 16 / kFNT;
+  const uint32_t nvec = static_cast<uint32_t>((stop - base + 15) / 16);
+  uint4 v[kVecs];
+#pragma unroll
+  for (int j = 0; j < kVecs; ++j) {
+    const uint32_t i = tid + j * kFNT;
+    const uint64_t off = base + 16ull * i;
+    v[j] = make_uint4(0, 0, 0, 0);
+    if (i < nvec) {
       if (off + 16 <= bytes) {
-        s_text[v] = *reinterpret_cast<const uint4*>(text + off);
+        v[j] = *reinterpret_cast<const uint4*>(text + off);
       } else {
         uint32_t w[4] = {0, 0, 0, 0};
         for (int b = 0; off + b < bytes && b < 16; ++b)
           w[b >> 2] |= static_cast<uint32_t>(text[off + b]) << (8 * (b & 3));
-        s_text[v] = make_uint4(w[0], w[1], w[2], w[3]);
+        v[j] = make_uint4(w[0], w[1], w[2], w[3]);
       }
     }
   }
+  const uint32_t pat = 0x01010101u * delim;
+#pragma unroll
+  for (int j = 0; j < kVecs; ++j) {
+    const uint32_t i = tid + j * kFNT;
+    if (i < nvec) {
+      s_text[i] = v[j];
+      s_bits[i] = static_cast<uint16_t>(byte_bits16(v[j], pat));
+    }
+  }
   __syncthreads();
-  const uint64_t r = r0 + threadIdx.x;
-  if (r >= rows) return;
-  const uint64_t pos = r == 0 ? 0 : ends[r - 1] + 1;
-  const uint64_t end = r < n_newlines ? ends[r] : bytes;
-  if (staged) {
-    const uint8_t* lds = reinterpret_cast<const uint8_t*>(s_text);
-    // The delimiter search reads 8 aligned bytes of LDS at a time: the
-    // lowest flagged byte of (x - 0x01..01) & ~x & 0x80..80 is x's first
-    // zero byte, x being the word XOR the delimiter in every byte.
-    const uint64_t pat = 0x0101010101010101ull * delim;
-    auto scan = [&](uint64_t q, uint64_t e) -> uint64_t {
-      uint32_t i = static_cast<uint32_t>(q - base);
-      const uint32_t ie = static_cast<uint32_t>(e - base);
-      while (i < ie && (i & 7u)) {
-        if (lds[i] == delim) return base + i;
-        ++i;
+  const uint8_t* lds = reinterpret_cast<const uint8_t*>(s_text);
+  if (mine) {
+    const uint32_t p = static_cast<uint32_t>(pos - base);
+    uint32_t e = static_cast<uint32_t>(end - base);
+    if (e > p && lds[e - 1] == '\r') --e;
+    s_start[tid] = static_cast<uint16_t>(p);
+    const uint64_t* bits = reinterpret_cast<const uint64_t*>(s_bits);
+    uint32_t word = p >> 6;
+    uint64_t m = bits[word] & (~0ull << (p & 63));
+    int f = 0;
+    for (;;) {
+      while (!m && (word + 1) * 64 < e) m = bits[++word];
+      const uint32_t d0 = m ? word * 64 + static_cast<uint32_t>(__builtin_ctzll(m)) : e;
+      const uint32_t d = d0 < e ? d0 : e;
+      s_ends[f * kFRows + tid] = static_cast<uint16_t>(d);
+      if (++f == tasks.fields) break;
+      if (d == e) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(short_rows), 1ull);
+        for (; f < tasks.fields; ++f) s_ends[f * kFRows + tid] = kNoField;
+        break;
       }
-      for (; i + 8 <= ie; i += 8) {
-        const uint64_t x = *reinterpret_cast<const uint64_t*>(lds + i) ^ pat;
-        const uint64_t z = (x - 0x0101010101010101ull) & ~x & 0x8080808080808080ull;
-        if (z) return base + i + (static_cast<uint32_t>(__builtin_ctzll(z)) >> 3);
+      m &= m - 1;
+    }
+  }
+  __syncthreads();
+  constexpr int kHalves = kFRows / kWave;
+  for (int c = static_cast<int>(wave_id()); c < tasks.n * kHalves; c += kFNT / kWave) {
+    const int f = tasks.f[c / kHalves];
+    const uint32_t row = static_cast<uint32_t>(c % kHalves) * kWave + lane_id();
+    if (r0 + row >= rows) continue;
+    const uint32_t fe = s_ends[f * kFRows + row];
+    int64_t iv = 0;
+    double dv = 0.0;
+    if (fe != kNoField) {  // missing fields read 0
+      const uint32_t fs = f ? s_ends[(f - 1) * kFRows + row] + 1u : s_start[row];
+      const int t = cols.t[f];
+      if (t == RFX_TBL_STR) {
+        // The field's address; its end (delimiter, '\r' or newline) becomes
+        // its terminating NUL.  A field running to the end of the text has
+        // nowhere to end: it reads as the null pointer (the empty string).
+        if (base + fe < bytes) {
+          iv = static_cast<int64_t>(reinterpret_cast<uintptr_t>(text + base + fs));
+          text[base + fe] = 0;
+        }
+      } else {
+        parse_staged(s_text, fs, fe, t, &iv, &dv);
       }
-      while (i < ie && lds[i] != delim) ++i;
-      return base + i;
-    };
-    parse_row([&](uint64_t q) -> uint8_t { return lds[q - base]; }, scan, text, bytes, r, pos,
-              end, n_fields, cols, short_rows);
-  } else {
-    auto scan = [&](uint64_t q, uint64_t e) -> uint64_t {
-      while (q < e && text[q] != delim) ++q;
-      return q;
-    };
-    parse_row([&](uint64_t q) -> uint8_t { return text[q]; }, scan, text, bytes, r, pos, end,
-              n_fields, cols, short_rows);
+    }
+    tbl_store(cols, f, r0 + row, iv, dv);
   }
 }
 
@@ -311,7 +568,7 @@ extern "C" int rfx_tbl_parse(rfx_ctx* ctx, void* text, uint64_t bytes, char deli
   }
   // Row ends are kept for the rows that are parsed (the count covers all).
   const uint64_t ntiles = bytes ? (bytes + kLTile - 1) / kLTile : 0;
-  const uint64_t ecap = capacity < bytes ? capacity + 1 : (bytes ? bytes : 1);
+  const uint64_t ecap = !capacity ? 1 : capacity < bytes ? capacity + 1 : (bytes ? bytes : 1);
   Carve c(nullptr);
   c.take<uint64_t>(ecap);
   c.take<uint64_t>(ntiles ? ntiles : 1);
@@ -327,7 +584,15 @@ extern "C" int rfx_tbl_parse(rfx_ctx* ctx, void* text, uint64_t bytes, char deli
                    (reinterpret_cast<char*>(counts + 2) - reinterpret_cast<char*>(status)) / 4, 0));
   RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(short_rows), 2, 0));
   if (!ntiles) RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(rows), 2, 0));
-  if (ntiles) {
+  if (ntiles && !capacity) {
+    RFX_PROF(ctx, "tbl.rows");
+    const uint64_t most = static_cast<uint64_t>(ctx->device_cus) * 4;
+    const uint64_t blocks = (bytes + 16 * kCNT - 1) / (16 * kCNT);
+    k_tbl_count<<<static_cast<uint32_t>(blocks < most ? blocks : most), kCNT, 0, ctx->stream>>>(
+        static_cast<const uint8_t*>(text), bytes, reinterpret_cast<uintptr_t>(text) % 16 == 0,
+        counts, rows, ticket);
+    RFX_LAUNCHED();
+  } else if (ntiles) {
     RFX_PROF(ctx, "tbl.rows");
     k_tbl_rows<<<static_cast<uint32_t>(ntiles), kLNT, 0, ctx->stream>>>(
         static_cast<const uint8_t*>(text), bytes, reinterpret_cast<uintptr_t>(text) % 16 == 0, ends,
@@ -343,9 +608,14 @@ extern "C" int rfx_tbl_parse(rfx_ctx* ctx, void* text, uint64_t bytes, char deli
   const uint64_t todo = n < capacity ? n : capacity;
   if (todo && n_fields) {
     RFX_PROF(ctx, "tbl.fields");
-    k_tbl_fields<<<static_cast<uint32_t>((todo + kFNT - 1) / kFNT), kFNT, 0, ctx->stream>>>(
+    TblTasks tasks{};
+    tasks.fields = n_fields;
+    for (int f = 0; f < n_fields; ++f)
+      if (types[f] != RFX_TBL_SKIP) tasks.f[tasks.n++] = static_cast<uint8_t>(f);
+    k_tbl_fields<<<static_cast<uint32_t>((todo + kFRows - 1) / kFRows), kFNT,
+                   n_fields * kFRows * sizeof(uint16_t), ctx->stream>>>(
         static_cast<uint8_t*>(text), bytes, reinterpret_cast<uintptr_t>(text) % 16 == 0,
-        ends, newlines, todo, static_cast<uint8_t>(delim), n_fields, cols, short_rows);
+        ends, newlines, todo, static_cast<uint8_t>(delim), tasks, cols, short_rows);
     RFX_LAUNCHED();
     RFX_HIP(hipStreamSynchronize(ctx->stream));
   }

@@ -26,11 +26,12 @@ def _call(ctx, text, nbytes, delim, spec, columns, capacity):
     types = (ctypes.c_int * max(len(spec), 1))(*[TBL[s] for s in spec])
     ptrs = (ctypes.c_void_p * max(len(spec), 1))(*[c.ptr if c is not None else None
                                                    for c in columns])
-    rows, short = rfx.u64_cell(), rfx.u64_cell()
+    cells = rfx.DeviceBuffer(16)  # rows, rows with missing fields: both are written
     rfx._check("rfx_tbl_parse", rfx.lib().rfx_tbl_parse(
         ctx.handle, text.ptr, nbytes, delim.encode(), types, len(spec), ptrs, capacity,
-        rows.ptr, short.ptr))
-    return rfx.read_u64(rows), rfx.read_u64(short)
+        cells.ptr, cells.ptr + 8))
+    rows, short = cells.download(np.uint64, 2)
+    return int(rows), int(short)
 
 
 def parse_tbl(ctx, text, spec: Sequence[str], delim: str = "|",

@@ -165,3 +165,29 @@ def test_freed_blocks_are_handed_out_again_whole(rf):
             live.append((buf, step % 251))
     for buf, tag in live:
         assert (buf.download(np.uint8) == tag).all()
+
+
+# Fields that the word-wise conversion takes and those it leaves to the byte
+# loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
+# 3 digits after them, letters inside; dates of other shapes; rows short of
+# fields; blocks whose text fits the stage and blocks whose text does not.
+# (Delimiters that keep the columns: an 11-digit year or a decimal past 2^64
+# overflows where the oracle's integers do not.)
+@pytest.mark.parametrize("wide", [0, 300])
+@pytest.mark.parametrize("delim", ["|", ","])
+def test_field_shapes_match_oracle(rf, ctx, wide, delim):
+    rng = np.random.default_rng(wide + len(delim))
+    ints = ["", "0", "7", "12345678", "123456789", "99999999999", "-5", "+5", " 42", "4 2", "1x", "x1",
+            "00000012", "2147483648", "12.5", "-", "18446744073709551616"]
+    decs = ["", "1.5", "12.25", "1234567.89", "12345678.9", "123456789.01", ".5", "5.", "1.234", "-1.25",
+            " 2.50", "1.2.3", "1e3", "12345678", "0.07", "0.1", "x", "1.x", "1.2x", "99999999.99"]
+    dates = ["1994-07-01", "1992-02-29", "1998-12-31", "94-7-1", "1994/07/01", "", "1994-07", "1994-07-0x",
+             " 1996-03-01", "1996-03-01 ", "+1995-+1-+2", "12345-01-01"]
+    rows = []
+    for i in range(1500):
+        f = [rng.choice(ints), rng.choice(decs), rng.choice(dates), rng.choice(ints), rng.choice(decs),
+             "A" * int(rng.integers(0, 3)), rng.choice(ints)]
+        rows.append(delim.join(f[: int(rng.choice([7, 7, 7, 7, 1, 4, 6]))]) + delim * int(rng.integers(0, 3))
+                    + "c" * int(rng.integers(0, wide + 1)) + ("\r" if i % 11 == 0 else ""))
+    text = ("\n".join(rows) + ("\n" if wide else "")).encode()
+    check(rf, ctx, text, ["i32", "f64", "date", "i64", "f64", "char", "u8"], delim)
