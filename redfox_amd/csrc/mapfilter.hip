@@ -78,6 +78,17 @@ __global__ __launch_bounds__(kMNT) void k_mapfilter(MfIn in, uint64_t n, rfx_mf_
       n, ntiles, n_kept, status, ticket);
 }
 
+// The same without a filter.
+__global__ __launch_bounds__(kMNT) void k_mapfilter_rows(MfIn in, uint64_t n, rfx_mf_program prog,
+                                                         MfOut out,
+                                                         uint64_t* __restrict__ n_kept) {
+  mapfilter_rows<1>([](uint64_t) { return Empty{}; },
+                    [&](uint64_t r, uint64_t pos, Empty) {
+                      run_ops(prog, 0, prog.n_ops, in, out, r, pos);
+                    },
+                    n, n_kept);
+}
+
 bool valid_col_type(int t) { return t >= RFX_MF_U8 && t <= RFX_MF_TUPLE16; }
 
 bool valid_code(uint32_t c) {
@@ -149,31 +160,35 @@ void jit_ops(std::string& s, const rfx_mf_program& p, uint32_t begin, uint32_t e
   }
 }
 
+// Rows per thread of the output phase.
+int jit_out_rows(const rfx_mf_program& p) {
+  uint32_t n_out_ops = 0;
+  for (uint32_t pc = p.n_filter; pc < p.n_ops; ++pc) n_out_ops += p.ops[pc].code == RFX_MF_OUT;
+  const uint32_t n_emit = p.n_ops - p.n_filter;
+  return (n_emit <= 24 && n_out_ops <= 4) ? 8 : (n_emit <= 48 && n_out_ops <= 8) ? 2 : 1;
+}
+
 // One kernel for a program with its column and output types.  Short
 // phases run their row batches unrolled (more loads in flight per wave);
 // long ones, or outputs with many values per row, keep fewer copies.
 std::string jit_source(const rfx_mf_program& p, const rfx_mf_col* cols, const rfx_mf_out* outs) {
   uint32_t n_out_ops = 0;
   for (uint32_t pc = p.n_filter; pc < p.n_ops; ++pc) n_out_ops += p.ops[pc].code == RFX_MF_OUT;
-  const uint32_t n_emit = p.n_ops - p.n_filter;
   const int uf = p.n_filter <= 24 ? 8 : p.n_filter <= 48 ? 2 : 1;
-  const int uo = (n_emit <= 24 && n_out_ops <= 4) ? 8 : (n_emit <= 48 && n_out_ops <= 8) ? 2 : 1;
+  const int uo = jit_out_rows(p);
   std::string s =
       "#include \"mapfilter_dev.h\"\n"
       "using namespace rfx;\n"
       "struct Vals { uint64_t v[" + std::to_string(n_out_ops ? n_out_ops : 1) + "]; };\n"
       "extern \"C\" __global__ __launch_bounds__(kMNT) void rfx_mf_jit(\n"
       "    MfIn in, MfOut out, uint64_t n, uint32_t ntiles, uint64_t* __restrict__ n_kept,\n"
-      "    uint64_t* __restrict__ status, uint32_t* __restrict__ ticket) {\n"
-      "  auto filter = [&](uint64_t row) -> bool {\n";
-  if (p.n_filter == 0) {
-    s += "    return true;\n";
-  } else {
-    s += "    uint64_t R[16] = {};\n";
+      "    uint64_t* __restrict__ status, uint32_t* __restrict__ ticket) {\n";
+  if (p.n_filter) {
+    s += "  auto filter = [&](uint64_t row) -> bool {\n    uint64_t R[16] = {};\n";
     jit_ops(s, p, 0, p.n_filter, cols);
-    s += "    return R[" + std::to_string(p.keep_reg) + "] != 0;\n";
+    s += "    return R[" + std::to_string(p.keep_reg) + "] != 0;\n  };\n";
   }
-  s += "  };\n  auto compute = [&](uint64_t row) -> Vals {\n    Vals o{};\n    uint64_t R[16] = {};\n";
+  s += "  auto compute = [&](uint64_t row) -> Vals {\n    Vals o{};\n    uint64_t R[16] = {};\n";
   jit_ops(s, p, p.n_filter, p.n_ops, cols);
   s += "    return o;\n  };\n  auto store = [&](uint64_t, uint64_t pos, const Vals& o) {\n";
   char line[128];
@@ -185,8 +200,11 @@ std::string jit_source(const rfx_mf_program& p, const rfx_mf_col* cols, const rf
                   outs[op.b].type, slot++);
     s += line;
   }
-  s += "  };\n  mapfilter_tile<" + std::to_string(uf) + ", " + std::to_string(uo) +
-       ">(filter, compute, store, n, ntiles, n_kept, status, ticket);\n}\n";
+  if (p.n_filter)
+    s += "  };\n  mapfilter_tile<" + std::to_string(uf) + ", " + std::to_string(uo) +
+         ">(filter, compute, store, n, ntiles, n_kept, status, ticket);\n}\n";
+  else
+    s += "  };\n  mapfilter_rows<" + std::to_string(uo) + ">(compute, store, n, n_kept);\n}\n";
   return s;
 }
 
@@ -343,6 +361,25 @@ extern "C" int rfx_mapfilter(rfx_ctx* ctx, const rfx_mf_col* cols, int n_cols, u
     }
   }
   if (n_rows == 0) return fill_u32(ctx, reinterpret_cast<uint32_t*>(n_kept), 2, 0);
+  if (prog->n_filter == 0) {
+    const uint64_t per_block = static_cast<uint64_t>(kMNT) * (fn ? jit_out_rows(*prog) : 1);
+    uint64_t blocks = (n_rows + per_block - 1) / per_block;
+    if (blocks > (1u << 20)) blocks = 1u << 20;
+    RFX_PROF(ctx, "mapfilter");
+    if (fn) {
+      uint32_t none = 0;
+      uint64_t* status = nullptr;
+      uint32_t* ticket = nullptr;
+      void* args[] = {&in, &out, &n_rows, &none, &n_kept, &status, &ticket};
+      RFX_HIP(hipModuleLaunchKernel(fn, static_cast<uint32_t>(blocks), 1, 1, kMNT, 1, 1, 0,
+                                    ctx->stream, args, nullptr));
+      return RFX_OK;
+    }
+    k_mapfilter_rows<<<static_cast<uint32_t>(blocks), kMNT, 0, ctx->stream>>>(in, n_rows, *prog,
+                                                                              out, n_kept);
+    RFX_LAUNCHED();
+    return RFX_OK;
+  }
   const uint64_t ntiles = (n_rows + kMTile - 1) / kMTile;
   Carve c(nullptr);
   c.take<uint64_t>(ntiles);

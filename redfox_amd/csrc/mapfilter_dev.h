@@ -392,4 +392,36 @@ __device__ __forceinline__ void mapfilter_tile(Filter filter, Compute compute, S
   }
 }
 
+// A program without a filter keeps every row at its own position: no
+// compaction, no ticket and no look-back (and no launch to clear their
+// words).  A block computes UO rows per thread before it stores any.  The
+// Q1 plan over 4.2 M rows runs 36 such passes of its 39: 3.83 -> 3.50 ms.
+template <int UO, class Compute, class Store>
+__device__ __forceinline__ void mapfilter_rows(Compute compute, Store store, uint64_t n,
+                                               uint64_t* n_kept) {
+  constexpr uint64_t kRows = static_cast<uint64_t>(kMNT) * UO;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *n_kept = n;
+  for (uint64_t base = blockIdx.x * kRows; base < n; base += gridDim.x * kRows) {
+    decltype(compute(base)) v[UO];
+    const uint64_t r0 = base + threadIdx.x;
+    if (base + kRows <= n) {  // uniform
+#pragma unroll
+      for (int u = 0; u < UO; ++u) v[u] = compute(r0 + u * kMNT);
+#pragma unroll
+      for (int u = 0; u < UO; ++u) store(r0 + u * kMNT, r0 + u * kMNT, v[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < UO; ++u) {
+        const uint64_t r = r0 + u * kMNT;
+        v[u] = compute(r < n ? r : n - 1);
+      }
+#pragma unroll
+      for (int u = 0; u < UO; ++u) {
+        const uint64_t r = r0 + u * kMNT;
+        if (r < n) store(r, r, v[u]);
+      }
+    }
+  }
+}
+
 }  // namespace rfx

@@ -82,6 +82,22 @@ def test_sizes_and_order(rf, mctx, orc, n):
     run(rf, mctx, orc, [v.view(np.int64), rows], ["i64", "u64"], build, n)
 
 
+# Programs without a filter: one row to past a block of 8, 2 and 1 rows per
+# thread (few, several and many outputs).
+@pytest.mark.parametrize("n", [1, 511, 513, 1024, 1025, 4095, 4097, (1 << 20) + 5])
+@pytest.mark.parametrize("outs", [2, 6, 8])
+def test_rows_without_filter(rf, mctx, orc, n, outs):
+    v = datagen.splitmix64(17 + n, n).view(np.int64)
+    w = datagen.u32(18 + n, n)
+
+    def build(x, a, b):
+        for k in range(outs):
+            x.emit(a * (k + 1) + b - (a % (k + 2)) * (b + k), ["i64", "u8", "i32", "f64"][k % 4])
+
+    kept, _ = run(rf, mctx, orc, [v, w], ["i64", "u32"], build, n)
+    assert kept == n
+
+
 def test_keep_all_and_none(rf, mctx, orc):
     v = np.arange(50_000, dtype=np.int32)
     run(rf, mctx, orc, [v], ["i32"], lambda x, a: x.emit(a * 3, "i64"))
