@@ -46,18 +46,12 @@ __device__ __forceinline__ void store_w(void* base, uint64_t i, int w, u128 v) {
 }
 
 // Number of A elements among the first `diag` merged elements when A wins
-// ties (A[i] <= B[j] puts A[i] first).
-template <class K>
+// ties (A[i] <= B[j] puts A[i] first), by G lanes.
+template <uint32_t G, class K>
 __device__ __forceinline__ uint64_t merge_path_lower(const K* a, uint64_t na, const K* b,
                                                      uint64_t nb, uint64_t diag) {
-  uint64_t lo = diag > nb ? diag - nb : 0;
-  uint64_t hi = diag < na ? diag : na;
-  while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    if (!lt(b[diag - 1 - mid], a[mid])) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
+  return group_search<G>(diag > nb ? diag - nb : 0, diag < na ? diag : na,
+                      [&](uint64_t mid) { return !lt(b[diag - 1 - mid], a[mid]); });
 }
 
 // ---------------------------------------------------------------------------
@@ -70,16 +64,22 @@ __device__ __forceinline__ uint64_t merge_path_lower(const K* a, uint64_t na, co
 constexpr int kFbNV = RFX_FB_NV;
 constexpr int kFbNT = 256;
 
-template <class K>
+template <uint32_t G, class K>
 __global__ __launch_bounds__(256) void k_fb_partition(const K* __restrict__ a, uint64_t na,
                                                       const K* __restrict__ b, uint64_t nb,
                                                       uint64_t ntiles, uint32_t nv,
-                                                      uint64_t* __restrict__ split) {
-  uint64_t t = blockIdx.x * 256ull + threadIdx.x;
+                                                      uint64_t* __restrict__ split,
+                                                      uint32_t* __restrict__ zero,
+                                                      uint32_t zero_words) {
+  // The search kernel's status words and ticket are cleared here.
+  const uint64_t x = blockIdx.x * 256ull + threadIdx.x;
+  if (x < zero_words) zero[x] = 0;
+  const uint64_t t = x / G;
   if (t > ntiles) return;
   uint64_t diag = t * nv;
   if (diag > na + nb) diag = na + nb;
-  split[t] = merge_path_lower(a, na, b, nb, diag);
+  const uint64_t s = merge_path_lower<G>(a, na, b, nb, diag);
+  if (x % G == 0) split[t] = s;
 }
 
 // The largest key of each width: the sentinel that follows a tile's right
@@ -388,32 +388,32 @@ __global__ __launch_bounds__(NT * kFbSub, 8) void k_find_bounds(
 // starts (B = left_count, non-decreasing).  A row start s comes before
 // output g when s <= g, so output g belongs to the last row started.
 // ---------------------------------------------------------------------------
+template <uint32_t G>
 __device__ __forceinline__ uint64_t merge_path_rows(const int32_t* starts, uint64_t nrows,
                                                     uint64_t total, uint64_t diag) {
-  uint64_t lo = diag > nrows ? diag - nrows : 0;
-  uint64_t hi = diag < total ? diag : total;
-  while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    uint64_t s = static_cast<uint32_t>(starts[diag - 1 - mid]);
-    if (mid < s) lo = mid + 1;  // output mid precedes the row start
-    else hi = mid;
-  }
-  return lo;  // number of outputs among the first diag merged items
+  // Number of outputs among the first diag merged items: output mid goes
+  // first where it precedes the row start.
+  return group_search<G>(diag > nrows ? diag - nrows : 0, diag < total ? diag : total,
+                      [&](uint64_t mid) {
+                        return mid < static_cast<uint32_t>(starts[diag - 1 - mid]);
+                      });
 }
 
+template <uint32_t G>
 __global__ __launch_bounds__(256) void k_expand_partition(const int32_t* __restrict__ starts,
                                                           uint64_t nrows,
                                                           const uint64_t* __restrict__ total_p,
                                                           uint64_t total_cap, uint64_t ntiles_cap,
                                                           uint32_t nv,
                                                           uint64_t* __restrict__ split) {
-  uint64_t t = blockIdx.x * 256ull + threadIdx.x;
+  const uint64_t x = blockIdx.x * 256ull + threadIdx.x, t = x / G;
   if (t > ntiles_cap) return;
   // Never expand past the caller's capacity, whatever the device says.
   const uint64_t total = *total_p < total_cap ? *total_p : total_cap;
   uint64_t diag = t * nv;
   if (diag > total + nrows) diag = total + nrows;
-  split[t] = merge_path_rows(starts, nrows, total, diag);
+  const uint64_t s = merge_path_rows<G>(starts, nrows, total, diag);
+  if (x % G == 0) split[t] = s;
 }
 
 // Output g of the tile gets (row, right index).  Mode 0 writes the index
@@ -703,11 +703,16 @@ int find_bounds_nv(rfx_ctx* ctx, int32_t* lb, int32_t* lc, uint64_t* total, cons
   const uint64_t nblk = fb_blocks(ntiles);
   uint64_t* status = w.take<uint64_t>(nblk);
   uint32_t* ticket = w.take<uint32_t>(1);
-  // status and ticket are adjacent after alignment; zero both.
-  RFX_TRY(fill_u32(ctx, reinterpret_cast<uint32_t*>(status),
-                   (reinterpret_cast<char*>(ticket + 1) - reinterpret_cast<char*>(status)) / 4, 0));
-  k_fb_partition<K><<<static_cast<uint32_t>((ntiles + 1 + 255) / 256), 256, 0, ctx->stream>>>(
-      static_cast<const K*>(left), nl, static_cast<const K*>(right), nr, ntiles, NV, split);
+  // status and ticket are adjacent after alignment: both are cleared by the
+  // split kernel: their words are at most 2 per block of 4 tiles and 65 of
+  // alignment, fewer than its threads.
+  const uint32_t words = static_cast<uint32_t>(
+      (reinterpret_cast<char*>(ticket + 1) - reinterpret_cast<char*>(status)) / 4);
+  const auto partition = ntiles <= kGroupTiles ? k_fb_partition<kSearchLanes, K>
+                                               : k_fb_partition<1, K>;
+  partition<<<split_blocks(ntiles), 256, 0, ctx->stream>>>(
+      static_cast<const K*>(left), nl, static_cast<const K*>(right), nr, ntiles, NV, split,
+      reinterpret_cast<uint32_t*>(status), words);
   RFX_LAUNCHED();
   const bool prof = own && ctx->profiling;
   if (prof) prof_begin(ctx, "join.find_bounds");
@@ -783,8 +788,10 @@ int expand_nv(rfx_ctx* ctx, int mode, int32_t* li, int32_t* ri, const GatherSpec
   RFX_TRY(ensure_workspace(ctx, c.off));
   Carve w(ctx->ws);
   uint64_t* split = w.take<uint64_t>(ntiles + 1);
-  k_expand_partition<<<static_cast<uint32_t>((ntiles + 1 + 255) / 256), 256, 0, ctx->stream>>>(
-      lc, nl, total, total_cap, ntiles, NV, split);
+  const auto partition =
+      ntiles <= kGroupTiles ? k_expand_partition<kSearchLanes> : k_expand_partition<1>;
+  partition<<<split_blocks(ntiles), 256, 0, ctx->stream>>>(lc, nl, total, total_cap, ntiles, NV,
+                                                           split);
   RFX_LAUNCHED();
   RFX_PROF(ctx, mode == 0 ? "join.expand" : mode == 1 ? "join.expand_gather" : "join.expand_project");
   // Sources wider than 8 bytes take the 128-bit register form.

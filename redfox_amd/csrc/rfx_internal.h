@@ -105,6 +105,13 @@ int ctx_cells(rfx_ctx* ctx, uint64_t** cells);
 // (graph-capture safe, unlike hipMemsetAsync).
 int fill_u32(rfx_ctx* ctx, uint32_t* p, uint64_t words, uint32_t value);
 
+// Kernels that find the splits before tiles 0 .. ntiles take 8 threads per
+// split (group_search) up to kGroupTiles tiles, one beyond; blocks of 256.
+constexpr uint64_t kGroupTiles = 8192;
+inline uint32_t split_blocks(uint64_t ntiles) {
+  return static_cast<uint32_t>(((ntiles <= kGroupTiles ? 8 : 1) * (ntiles + 1) + 255) / 256);
+}
+
 // Type-code helpers (RelationalAlgebraKernel.h:81-95).
 inline int bytes_of_type(uint64_t type) {
   switch (type) {

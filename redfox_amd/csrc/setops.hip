@@ -32,17 +32,11 @@ constexpr int kSNT = 256;
 constexpr int kSVT = 8;
 constexpr int kSNV = kSNT * kSVT;
 
-template <class K>
+template <uint32_t G, class K>
 __device__ __forceinline__ uint64_t mp_lower(const K* a, uint64_t na, const K* b, uint64_t nb,
                                              uint64_t diag) {
-  uint64_t lo = diag > nb ? diag - nb : 0;
-  uint64_t hi = diag < na ? diag : na;
-  while (lo < hi) {
-    uint64_t mid = (lo + hi) >> 1;
-    if (!lt(b[diag - 1 - mid], a[mid])) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
+  return group_search<G>(diag > nb ? diag - nb : 0, diag < na ? diag : na,
+                      [&](uint64_t mid) { return !lt(b[diag - 1 - mid], a[mid]); });
 }
 
 // Element shuffles across the wave (lane - delta / lane + delta; a lane
@@ -72,16 +66,17 @@ __device__ __forceinline__ K shfl_down_elem(K v, int delta) {
   }
 }
 
-template <class K>
+template <uint32_t G, class K>
 __global__ __launch_bounds__(256) void k_set_partition(const K* __restrict__ a, uint64_t na,
                                                        const K* __restrict__ b, uint64_t nb,
                                                        uint64_t ntiles, uint32_t nv,
                                                        uint64_t* __restrict__ split) {
-  uint64_t t = blockIdx.x * 256ull + threadIdx.x;
+  const uint64_t x = blockIdx.x * 256ull + threadIdx.x, t = x / G;
   if (t > ntiles) return;
   uint64_t diag = t * nv;
   if (diag > na + nb) diag = na + nb;
-  split[t] = mp_lower(a, na, b, nb, diag);
+  const uint64_t s = mp_lower<G>(a, na, b, nb, diag);
+  if (x % G == 0) split[t] = s;
 }
 
 // A view of one input: LDS for the tile's window [w0, w1), global elsewhere.
@@ -513,8 +508,9 @@ int set_op_impl(rfx_ctx* ctx, int op, void* out, uint64_t* n_out, uint64_t mul, 
   RFX_TRY(lb_workspace(ctx, ntiles, 0, &w, nullptr));
   const K* A = static_cast<const K*>(a);
   const K* B = static_cast<const K*>(b);
-  k_set_partition<K><<<static_cast<uint32_t>((ntiles + 1 + 255) / 256), 256, 0, ctx->stream>>>(
-      A, na, B, nb, ntiles, NV, w.split);
+  const auto partition = ntiles <= kGroupTiles ? k_set_partition<kSearchLanes, K>
+                                               : k_set_partition<1, K>;
+  partition<<<split_blocks(ntiles), 256, 0, ctx->stream>>>(A, na, B, nb, ntiles, NV, w.split);
   RFX_LAUNCHED();
   const uint32_t g = static_cast<uint32_t>(ntiles);
   K* O = static_cast<K*>(out);

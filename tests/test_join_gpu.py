@@ -303,3 +303,36 @@ def test_config1_plan_replayed_from_a_graph(rf, ctx, orc):
     g.close()
     gctx.close()
     stream.close()
+
+
+@pytest.mark.parametrize("extra", [0, 1])
+def test_splits_by_eight_lanes_and_by_one(rf, ctx, extra):
+    """find_bounds and the expansion over 8,192 tiles, the last whose splits
+    take eight lanes each, and over 8,193 (tiles of 2048)."""
+    nl = 3_000_000
+    nr = 8192 * 2048 - nl + extra
+    rng = np.random.default_rng(extra)
+    left = np.sort(rng.integers(0, 1 << 23, nl).astype(np.uint32))
+    right = np.sort(rng.integers(0, 1 << 23, nr).astype(np.uint32))
+    L, R = rf.DeviceBuffer.from_numpy(left), rf.DeviceBuffer.from_numpy(right)
+    lb, lc, tot = rf.DeviceBuffer(4 * nl), rf.DeviceBuffer(4 * nl), rf.u64_cell()
+    try:
+        ctx.tune("join.fb_tile", 2048)
+        ctx.join_find_bounds(lb, lc, tot, L, nl, R, nr, 4)
+    finally:
+        ctx.tune("join.fb_tile", 0)
+    lo = np.searchsorted(right, left, "left")
+    cnt = np.searchsorted(right, left, "right") - lo
+    total = int(cnt.sum())
+    assert rf.read_u64(tot) == total
+    assert np.array_equal(lb.download(np.int32, nl), lo)
+    start = np.cumsum(cnt) - cnt
+    assert np.array_equal(lc.download(np.int32, nl), start)
+    for cap in (total, 8192 * 4096 - nl + extra):  # a capacity sets the expansion's tiles
+        out = [rf.DeviceBuffer(4 * max(cap, total)) for _ in range(2)]
+        ctx.join_main(out[0], out[1], tot, cap, lb, lc, nl)
+        rows = np.repeat(np.arange(nl), cnt)
+        m = min(cap, total)
+        assert np.array_equal(out[0].download(np.int32, m), rows[:m])
+        assert np.array_equal(out[1].download(np.int32, m),
+                              (lo[rows] + np.arange(total) - start[rows])[:m])

@@ -92,7 +92,7 @@ def test_rows_without_filter(rf, mctx, orc, n, outs):
 
     def build(x, a, b):
         for k in range(outs):
-            x.emit(a * (k + 1) + b - (a % (k + 2)) * (b + k), ["i64", "u8", "i32", "f64"][k % 4])
+            x.emit(a * (k + 1) - (b + k), ["i64", "u8", "i32", "f64"][k % 4])
 
     kept, _ = run(rf, mctx, orc, [v, w], ["i64", "u32"], build, n)
     assert kept == n
