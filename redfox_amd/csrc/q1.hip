@@ -7,8 +7,8 @@
 // shipdate <= cutoff, disc_price = price * (1 - disc), charge = disc_price *
 // (1 + tax), COUNT and TOTAL grouped by (returnflag, linestatus) - reads each
 // of the seven columns once (34 bytes per row) and keeps the six groups'
-// partial sums in registers.  Rows are dealt to a fixed grid (kQBlocks x
-// 256 threads, four consecutive rows per step), and the partials are
+// partial sums in registers.  Rows are dealt to a grid fixed by n
+// (four consecutive rows per step), and the partials are
 // combined by fixed trees, so the FP64 sums depend on n alone.
 #include "rfx_device.h"
 #include "rfx_internal.h"
@@ -17,7 +17,15 @@ namespace rfx {
 namespace {
 
 constexpr int kQNT = 256;
+// Blocks: 16 rows a thread, up to 2048 blocks (a function of n alone, as the
+// order of the sums is).  Every block reduces 36 values over its waves, so a
+// small n with 2048 blocks was all reduction: 4 M rows 55 -> 43 us, 100,000 46 -> 24 (with the averages made by
+// the last kernel instead of one more).
 constexpr uint32_t kQBlocks = 2048;
+constexpr uint32_t q1_blocks(uint64_t n) {
+  const uint64_t b = (n + 16 * 256 - 1) / (16 * 256);
+  return static_cast<uint32_t>(b < 1 ? 1 : b < kQBlocks ? b : kQBlocks);
+}
 constexpr int kQGroups = 6;
 constexpr int kQSums = 5;  // qty, base price, disc price, charge, disc
 
@@ -58,7 +66,7 @@ __global__ __launch_bounds__(kQNT) void k_q1_partial(
     a.c[k] = 0;
   }
   const uint64_t gtid = blockIdx.x * static_cast<uint64_t>(kQNT) + threadIdx.x;
-  const uint64_t stride = static_cast<uint64_t>(kQBlocks) * kQNT;
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kQNT;
   // Four consecutive rows per step: 16-byte loads of the 4-byte columns,
   // 4-byte loads of the byte columns, 2 x 16 bytes of each double column.
   const uint64_t n4 = n / 4;
@@ -101,30 +109,30 @@ __global__ __launch_bounds__(kQNT) void k_q1_partial(
   }
 }
 
-// One block per aggregate value: a fixed tree over the kQBlocks partials.
-__global__ __launch_bounds__(1024) void k_q1_final(const double* __restrict__ part,
+// One block per group: a fixed tree over the blocks' partials of each of its
+// six values, then the group's averages.
+__global__ __launch_bounds__(1024) void k_q1_final(const double* __restrict__ part, uint32_t nb,
                                                    double* __restrict__ out) {
-  __shared__ double sm[1024];
-  const uint32_t v = blockIdx.x;  // k * 6 + f
-  const double* p = part + static_cast<uint64_t>(v) * kQBlocks;
-  sm[threadIdx.x] = p[threadIdx.x] + p[threadIdx.x + 1024];
+  constexpr int NV = kQSums + 1;
+  __shared__ double sm[NV][1024];
+  const uint32_t t = threadIdx.x, k = blockIdx.x;
+#pragma unroll
+  for (int f = 0; f < NV; ++f) {
+    const double* p = part + static_cast<uint64_t>(k * NV + f) * kQBlocks;
+    sm[f][t] = (t < nb ? p[t] : 0.0) + (t + 1024 < nb ? p[t + 1024] : 0.0);
+  }
   __syncthreads();
-  for (int d = 512; d > 0; d >>= 1) {
-    if (threadIdx.x < static_cast<uint32_t>(d)) sm[threadIdx.x] += sm[threadIdx.x + d];
+  for (uint32_t d = 512; d > 0; d >>= 1) {
+    if (t < d) {
+#pragma unroll
+      for (int f = 0; f < NV; ++f) sm[f][t] += sm[f][t + d];
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const int k = v / (kQSums + 1), f = v % (kQSums + 1);
-    out[k * 8 + f] = sm[0];
-  }
-}
-
-__global__ void k_q1_avgs(double* __restrict__ out) {
-  const int k = threadIdx.x;
-  if (k < kQGroups) {
-    const double c = out[k * 8 + 5];
-    out[k * 8 + 6] = c > 0 ? out[k * 8 + 0] / c : 0.0;
-    out[k * 8 + 7] = c > 0 ? out[k * 8 + 1] / c : 0.0;
+  if (t < NV) out[k * 8 + t] = sm[t][0];
+  if (t < 2) {
+    const double c = sm[kQSums][0];
+    out[k * 8 + 6 + t] = c > 0 ? sm[t][0] / c : 0.0;
   }
 }
 
@@ -155,13 +163,11 @@ extern "C" int rfx_q1(rfx_ctx* ctx, double* out, const int32_t* shipdate,
   double* part = w.take<double>(static_cast<uint64_t>(kQGroups) * (kQSums + 1) * kQBlocks);
   {
     RFX_PROF(ctx, "q1.partial");
-    k_q1_partial<<<kQBlocks, kQNT, 0, ctx->stream>>>(shipdate, returnflag, linestatus, qty, price,
+    k_q1_partial<<<q1_blocks(n), kQNT, 0, ctx->stream>>>(shipdate, returnflag, linestatus, qty, price,
                                                        disc, tax, n, cutoff, part);
     RFX_LAUNCHED();
   }
-  k_q1_final<<<kQGroups * (kQSums + 1), 1024, 0, ctx->stream>>>(part, out);
-  RFX_LAUNCHED();
-  k_q1_avgs<<<1, 64, 0, ctx->stream>>>(out);
+  k_q1_final<<<kQGroups, 1024, 0, ctx->stream>>>(part, q1_blocks(n), out);
   RFX_LAUNCHED();
   return RFX_OK;
 }

@@ -131,7 +131,7 @@ def run_q1(rf, ctx, cols, cutoff):
     return out.download(np.float64, 48).reshape(6, 8)
 
 
-@pytest.mark.parametrize("n", [1, 3, 1000, 1_000_003])
+@pytest.mark.parametrize("n", [0, 1, 3, 1000, 4095, 4097, 8193, 1_000_003, 4_200_001, 8_392_705])
 def test_q1_matches_oracle(rf, ctx, orc, n):
     cols = datagen.lineitem(datagen.BASE_SEED + 2, n)
     got = run_q1(rf, ctx, cols, 2436)
