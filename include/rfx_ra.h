@@ -99,6 +99,10 @@ rfx_ctx* rfx_default_ctx(void);
 
 int rfx_device_count(int* count);
 int rfx_set_device(int device);
+/* rfx_free waits for the device, as hipFree does, and may keep the block
+ * (up to 64 MiB each, 512 MiB in all) for a later rfx_malloc; kept blocks go
+ * back to the runtime when an allocation fails and when a context is
+ * destroyed. */
 int rfx_malloc(void** ptr, uint64_t bytes);
 int rfx_free(void* ptr);
 int rfx_memcpy_htod(void* dst, const void* src, uint64_t bytes);
