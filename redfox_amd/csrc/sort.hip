@@ -192,7 +192,8 @@ __device__ __forceinline__ uint32_t sort_lookback_groups(const S* status, S* sum
 }
 
 // ---- tiles -----------------------------------------------------------------
-// The pass's blocks are persistent and take tiles until none is left.  With
+// The pass's blocks are persistent and take tiles until none is left, except
+// where there are as many as tiles and one ticket: then each takes one.  With
 // first == 0 every tile comes from one ticket.  Otherwise blocks are split
 // over kQueues queues by blockIdx, which the hardware deals out to the XCDs
 // in turn, and a queue hands out chunks of consecutive tiles (`first` tiles,
@@ -590,6 +591,8 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
   const uint32_t w = wave_id();
   const TileQueue<kChunkOf<TILE>> queue{ctrs + pass * kCtrWords, lists + pass * kQueues * list_len, list_len, first};
   if (tid == 0) s_tile = queue.tile(queue.ask());
+  // One tile per block: as many blocks as tiles, by the ticket.
+  const bool once = first == 0 && gridDim.x == ntiles;
   using SW = StatusWord<S>;
   S* st = status + (static_cast<uint64_t>(pass) * status_rows(ntiles)) * kBins;
 
@@ -754,7 +757,7 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
     // The next tile is asked for while this one is still being stored.
     uint32_t next = 0;
     if constexpr (VB == 0) {
-      if (tid == 0) s_tile = queue.tile(queue.ask());
+      if (tid == 0 && !once) s_tile = queue.tile(queue.ask());
     }
     if constexpr (VB > 0) {
       __syncthreads();  // every key is out of kbuf
@@ -765,7 +768,7 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
         if (FULL || idx < n) vbuf[(j & 1) ? (pos[j / 2] >> 16) : (pos[j / 2] & 0xFFFFu)] = vals[j];
       }
       __syncthreads();
-      if (tid == 0) next = queue.ask();
+      if (tid == 0 && !once) next = queue.ask();
 #pragma unroll
       for (int k = 0; k < IPT; ++k) {
         if (k % kScatterBatch == 0) __builtin_amdgcn_sched_barrier(0);
@@ -774,7 +777,7 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
           if (dst[k] < n32) vout[dst[k]] = vbuf[i];
         }
       }
-      if (tid == 0) s_tile = queue.tile(next);
+      if (tid == 0 && !once) s_tile = queue.tile(next);
     }
   };
   for (;;) {
@@ -789,6 +792,7 @@ __global__ __launch_bounds__(NT, 4) void k_onesweep(
     if (tile >= ntiles) break;
     if (static_cast<uint64_t>(tile) * TILE + TILE <= n) body(tile, std::true_type{});
     else body(tile, std::false_type{});
+    if (once) break;
   }
 
   // The last block to finish flips the buffer selector.  Every block read
@@ -920,8 +924,15 @@ int sort_impl(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
     return b;
   }();
   const uint64_t slots = static_cast<uint64_t>(ctx->device_cus) * per_cu;
-  const uint32_t grid = static_cast<uint32_t>(tiles < slots ? tiles : slots);
-  const uint32_t first = tiles > 2 * slots ? (grid + kQueues - 1) / kQueues : 0;
+  // A server's context (its workspace is the request's) shares the GPU with
+  // other requests' kernels: there each block takes one tile and gives its
+  // slot back, since blocks that stay until the pass ends keep the others
+  // waiting.  The saturated served mix: 1,103 requests/s with blocks that
+  // stay, 1,369 with one tile each (1,254 before there were any that stay);
+  // one request at a time, where nothing waits: 993 and 982.
+  const bool shared = ctx->ws_borrowed;
+  const uint32_t grid = static_cast<uint32_t>(tiles < slots || shared ? tiles : slots);
+  const uint32_t first = tiles > 2 * slots && !shared ? (grid + kQueues - 1) / kQueues : 0;
   for (int p = 0; p < passes; ++p) {
     RFX_PROF(ctx, "sort.onesweep");
     k_onesweep<KB, VB, NT, IPT, DB, LBW, S><<<grid, NT, 0, ctx->stream>>>(

@@ -263,3 +263,39 @@ def test_many_to_many_joins_match_numpy(served, rf, ctx):
             sink.close()
     for b in [bd, bg] + bufs3:
         b.close()
+
+
+@pytest.mark.parametrize("nf", [12 << 20, (14 << 20) + 5])
+def test_request_sorts_with_more_tiles_than_slots(rf, nf):
+    """Sorts of a request's relations with more tiles than the GPU holds
+    blocks at once (twice as many and more): each block takes one tile."""
+    from redfox_amd import serving as S
+
+    rng = np.random.default_rng(nf)
+    nd, groups = 50_000, 64
+    fk = rng.integers(0, nd, nf, dtype=np.uint32)
+    m = rng.integers(0, 1000, nf).astype(np.float64)  # sums are exact
+    dk, g = rng.permutation(nd).astype(np.uint32), rng.integers(0, groups, nd, dtype=np.uint32)
+    of_key = np.empty(nd, np.uint32)
+    of_key[dk] = g
+    row_g = of_key[fk]
+    exp = [np.arange(groups, dtype=np.uint32), np.bincount(row_g, m, groups),
+           np.bincount(row_g, minlength=groups).astype(np.uint32)]
+    srv = S.Server(0, slots=2, budget_bytes=4 << 30)
+    bufs = [rf.DeviceBuffer.from_numpy(x) for x in (fk, m, dk, g)]
+    rels = [S.Relation(), S.Relation()]
+    for rel, cols, rows, vbits in ((rels[0], bufs[:2], nf, 0), (rels[1], bufs[2:], nd, 6)):
+        rel.col[0], rel.col[1] = cols[0].ptr, cols[1].ptr
+        rel.rows, rel.key_bits, rel.val_bits = rows, 16, vbits
+    sid = srv.add_schema(1, rels)
+    sinks = [rf.DeviceBuffer(64 * 16) for _ in range(2)]
+    req = (S.Request * 2)()
+    for r, sink in zip(req, sinks):
+        r.schema, r.sink, r.sink_bytes = sid, sink.ptr, sink.nbytes
+    srv.run(req, S.MODE_CONTINUOUS)
+    for r, sink in zip(req, sinks):
+        assert r.status == 0 and r.rows == groups
+        check_sink(sink, r.rows, exp, [4, 8, 4], 64, 0)
+    srv.close()
+    for b in bufs + sinks:
+        b.close()
