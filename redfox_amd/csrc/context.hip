@@ -6,6 +6,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "block_cache.h"
 #include "rfx_device.h"
 #include "rfx_internal.h"
 
@@ -219,101 +220,37 @@ __global__ void k_gen_lineitem(int32_t* shipdate, uint8_t* flag, uint8_t* status
   }
 }
 
-// Blocks freed by rfx_free, kept for rfx_malloc: a text load allocates and
-// frees a column per field, each call of the runtime's allocator 10 to 40 us
-// (a million-row text load with 9 columns: 720 -> 500 us, with the passes over
-// the text).
-//
-// A block is kept only once the device is idle, as hipFree waits too: no
-// queued work of any stream or thread can still touch it, so it may be
-// handed to any of them.  Blocks of up to kKeepBlock bytes, kKeepTotal in
-// all; they go back to the runtime when an allocation fails and when a
-// context is destroyed.  Other pointers, other devices' blocks and frees
-// while a graph is being captured (no waiting then) go straight to the
-// runtime.
-class BlockCache {
- public:
-  int take(void** ptr, uint64_t bytes) {
-    const uint64_t size = rounded(bytes);
-    int dev = 0;
-    RFX_HIP(hipGetDevice(&dev));
-    if (size <= kKeepBlock) {
-      std::lock_guard<std::mutex> hold(mu_);
-      auto it = free_.find({dev, size});
-      if (it != free_.end()) {
-        *ptr = it->second.back();
-        it->second.pop_back();
-        if (it->second.empty()) free_.erase(it);
-        kept_ -= size;
-        out_[*ptr] = {dev, size};
-        return RFX_OK;
-      }
-    }
-    if (hipMalloc(ptr, size) != hipSuccess) {
-      (void)hipGetLastError();
-      drop();
-      if (hipMalloc(ptr, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(RFX_ENOMEM, "hipMalloc(%llu) failed", static_cast<unsigned long long>(bytes));
-      }
-      return RFX_OK;  // of its own size: not kept when freed
-    }
-    if (size <= kKeepBlock) {
-      std::lock_guard<std::mutex> hold(mu_);
-      out_[*ptr] = {dev, size};
-    }
-    return RFX_OK;
+// The runtime's side of the block cache.
+struct DeviceRuntime {
+  bool alloc(void** p, uint64_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
   }
-  // False: not a block to keep; the caller frees it.
-  bool give(void* ptr) {
-    std::pair<int, uint64_t> b;
-    {
-      std::lock_guard<std::mutex> hold(mu_);
-      auto it = out_.find(ptr);
-      if (it == out_.end()) return false;
-      b = it->second;
-      out_.erase(it);
-    }
-    int dev = 0;
-    if (g_capturing > 0 || hipGetDevice(&dev) != hipSuccess || dev != b.first ||
-        hipDeviceSynchronize() != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    std::lock_guard<std::mutex> hold(mu_);
-    if (kept_ + b.second > kKeepTotal) return false;
-    free_[b].push_back(ptr);
-    kept_ += b.second;
-    return true;
+  void release(void* p) { (void)hipFree(p); }
+  int device() {
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess) return dev;
+    (void)hipGetLastError();
+    return -1;
   }
-  void drop() {
-    std::map<std::pair<int, uint64_t>, std::vector<void*>> all;
-    {
-      std::lock_guard<std::mutex> hold(mu_);
-      all.swap(free_);
-      kept_ = 0;
-    }
-    for (auto& b : all)
-      for (void* p : b.second) (void)hipFree(p);
+  bool idle() {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
   }
-
- private:
-  static constexpr uint64_t kKeepBlock = 64ull << 20, kKeepTotal = 512ull << 20;
-  // Steps of an eighth of the size below, so that a block that held nearly
-  // as much is found again; sizes that are not kept stay as they are.
-  static uint64_t rounded(uint64_t bytes) {
-    if (bytes > kKeepBlock) return bytes;
-    uint64_t step = 256;
-    while (step * 16 < bytes) step *= 2;
-    return align_up(bytes, step);
+  uint64_t extent(void* p) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, p) == hipSuccess) return base == p ? size : 0;
+    (void)hipGetLastError();
+    return 0;
   }
-  std::mutex mu_;
-  std::map<std::pair<int, uint64_t>, std::vector<void*>> free_;
-  std::map<void*, std::pair<int, uint64_t>> out_;
-  uint64_t kept_ = 0;
+  bool capturing() { return g_capturing > 0; }
 };
 // Never destroyed: buffers may be freed by other objects' destructors.
-static BlockCache& g_blocks = *new BlockCache;
+using DeviceBlocks = BlockCache<DeviceRuntime>;
+static DeviceBlocks& g_blocks = *new DeviceBlocks;
 
 static uint32_t grid_for(uint64_t n) {
   uint64_t b = (n + 255) / 256;
@@ -511,10 +448,18 @@ int rfx_malloc(void** ptr, uint64_t bytes) {
   if (!ptr) return fail(RFX_EINVAL, "null pointer");
   *ptr = nullptr;
   if (bytes == 0) bytes = 1;
-  return g_blocks.take(ptr, bytes);
+  if (g_blocks.take(ptr, bytes)) return RFX_OK;
+  *ptr = nullptr;
+  return fail(RFX_ENOMEM, "hipMalloc(%llu) failed", static_cast<unsigned long long>(bytes));
 }
 int rfx_free(void* ptr) {
-  if (ptr && !g_blocks.give(ptr)) RFX_HIP(hipFree(ptr));
+  if (!ptr) return RFX_OK;
+  switch (g_blocks.give(ptr)) {
+    case DeviceBlocks::kKept: return RFX_OK;
+    case DeviceBlocks::kFreedBefore: return fail(RFX_EHIP, "rfx_free: %p is free already", ptr);
+    case DeviceBlocks::kCallerFrees: break;
+  }
+  RFX_HIP(hipFree(ptr));
   return RFX_OK;
 }
 int rfx_memcpy_htod(void* dst, const void* src, uint64_t bytes) {

@@ -167,6 +167,32 @@ def test_freed_blocks_are_handed_out_again_whole(rf):
         assert (buf.download(np.uint8) == tag).all()
 
 
+
+@pytest.mark.parametrize("size", [1000, 3 << 20, (64 << 20) + 1])
+def test_second_free_is_refused(rf, size):
+    """Freed twice: refused, whether the block is kept or the runtime's, and
+    the address is handed to one owner only."""
+    lib = rf.lib()
+
+    def get():
+        p = ctypes.c_void_p()
+        assert lib.rfx_malloc(ctypes.byref(p), size) == 0
+        return p.value
+
+    a = get()
+    assert lib.rfx_free(a) == 0
+    assert lib.rfx_free(a) != 0
+    b, c = get(), get()
+    assert b != c
+    for p, tag in ((b, 1), (c, 2)):
+        assert lib.rfx_memset(p, tag, size) == 0
+    host = np.empty(size, np.uint8)
+    for p, tag in ((b, 1), (c, 2)):
+        assert lib.rfx_memcpy_dtoh(host.ctypes.data, p, size) == 0
+        assert (host == tag).all()
+        assert lib.rfx_free(p) == 0
+
+
 # Fields that the word-wise conversion takes and those it leaves to the byte
 # loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
 # 3 digits after them, letters inside; dates of other shapes; rows short of
