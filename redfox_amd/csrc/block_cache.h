@@ -6,8 +6,8 @@
 // A block is kept only once the device is idle, as hipFree waits too: no
 // queued work of any stream or thread can still touch it, so it may be
 // handed to any of them.  Blocks of up to kKeepBlock bytes, kKeepTotal in
-// all; they go back to the runtime when an allocation fails and when a
-// context is destroyed.  Other pointers, other devices' blocks and frees
+// all; they go back to the runtime when an allocation fails (any of the
+// library's: alloc) and when a context is destroyed.  Other pointers, other devices' blocks and frees
 // while a graph is being captured (no waiting then) go straight to the
 // runtime.
 //
@@ -53,8 +53,7 @@ class BlockCache {
       }
     }
     if (!rt_.alloc(ptr, size)) {
-      drop();
-      if (!rt_.alloc(ptr, bytes)) return false;
+      if (!alloc(ptr, bytes)) return false;
       std::lock_guard<std::mutex> hold(mu_);
       blocks_.erase(*ptr);  // of its own size: not kept when freed
       return true;
@@ -63,6 +62,13 @@ class BlockCache {
     if (size <= kKeepBlock) blocks_[*ptr] = {dev, size, false};
     else blocks_.erase(*ptr);
     return true;
+  }
+
+  // Memory of the caller's own, which the caller releases: the kept blocks
+  // make room for it.  (Not while capturing: hipFree waits.)
+  bool alloc(void** ptr, uint64_t bytes) {
+    if (rt_.alloc(ptr, bytes)) return true;
+    return !rt_.capturing() && drop() && rt_.alloc(ptr, bytes);
   }
 
   // kFreedBefore: the block is kept already, so this is its second free.
@@ -92,8 +98,8 @@ class BlockCache {
     return kKept;
   }
 
-  // Gives every kept block back to the runtime.
-  void drop() {
+  // Gives every kept block back to the runtime; false if there was none.
+  bool drop() {
     std::vector<void*> all;
     {
       std::lock_guard<std::mutex> hold(mu_);
@@ -107,6 +113,7 @@ class BlockCache {
       kept_ = 0;
     }
     for (void* p : all) rt_.release(p);
+    return !all.empty();
   }
 
  private:

@@ -28,6 +28,44 @@ void die(const char* where, int status) {
   std::abort();
 }
 
+// The runtime's side of the block cache.
+struct DeviceRuntime {
+  bool alloc(void** p, uint64_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  void release(void* p) { (void)hipFree(p); }
+  int device() {
+    int dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess) return dev;
+    (void)hipGetLastError();
+    return -1;
+  }
+  bool idle() {
+    if (hipDeviceSynchronize() == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+  }
+  uint64_t extent(void* p) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, p) == hipSuccess) return base == p ? size : 0;
+    (void)hipGetLastError();
+    return 0;
+  }
+  bool capturing() { return g_capturing > 0; }
+};
+// Never destroyed: buffers may be freed by other objects' destructors.
+using DeviceBlocks = BlockCache<DeviceRuntime>;
+static DeviceBlocks& g_blocks = *new DeviceBlocks;
+
+bool device_alloc(void** ptr, uint64_t bytes) {
+  if (g_blocks.alloc(ptr, bytes)) return true;
+  *ptr = nullptr;
+  return false;
+}
+
 int ensure_workspace(rfx_ctx* ctx, uint64_t bytes) {
   if (bytes <= ctx->ws_bytes) return RFX_OK;
   if (ctx->capturing)
@@ -52,11 +90,9 @@ int ensure_workspace(rfx_ctx* ctx, uint64_t bytes) {
   }
   uint64_t want = align_up(bytes + bytes / 8, 1ull << 20);
   void* p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) {
-    (void)hipGetLastError();
+  if (!device_alloc(&p, want))
     return fail(RFX_ENOMEM, "workspace allocation of %llu bytes failed",
                 static_cast<unsigned long long>(want));
-  }
   ctx->ws = p;
   ctx->ws_bytes = want;
   return RFX_OK;
@@ -112,10 +148,8 @@ int ctx_cells(rfx_ctx* ctx, uint64_t** cells) {
     if (ctx->capturing) return fail(RFX_EINVAL, "context cells must be allocated before capture");
     RFX_HIP(hipSetDevice(ctx->device));
     void* p = nullptr;
-    if (hipMalloc(&p, kCtxCells * sizeof(uint64_t)) != hipSuccess) {
-      (void)hipGetLastError();
+    if (!device_alloc(&p, kCtxCells * sizeof(uint64_t)))
       return fail(RFX_ENOMEM, "allocating the context's scalar cells failed");
-    }
     ctx->cells = static_cast<uint64_t*>(p);
   }
   *cells = ctx->cells;
@@ -219,38 +253,6 @@ __global__ void k_gen_lineitem(int32_t* shipdate, uint8_t* flag, uint8_t* status
     tax[i] = static_cast<double>((b & 0xFFFF) % 9) / 100.0;
   }
 }
-
-// The runtime's side of the block cache.
-struct DeviceRuntime {
-  bool alloc(void** p, uint64_t bytes) {
-    if (hipMalloc(p, bytes) == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
-  }
-  void release(void* p) { (void)hipFree(p); }
-  int device() {
-    int dev = -1;
-    if (hipGetDevice(&dev) == hipSuccess) return dev;
-    (void)hipGetLastError();
-    return -1;
-  }
-  bool idle() {
-    if (hipDeviceSynchronize() == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
-  }
-  uint64_t extent(void* p) {
-    hipDeviceptr_t base = nullptr;
-    size_t size = 0;
-    if (hipMemGetAddressRange(&base, &size, p) == hipSuccess) return base == p ? size : 0;
-    (void)hipGetLastError();
-    return 0;
-  }
-  bool capturing() { return g_capturing > 0; }
-};
-// Never destroyed: buffers may be freed by other objects' destructors.
-using DeviceBlocks = BlockCache<DeviceRuntime>;
-static DeviceBlocks& g_blocks = *new DeviceBlocks;
 
 static uint32_t grid_for(uint64_t n) {
   uint64_t b = (n + 255) / 256;

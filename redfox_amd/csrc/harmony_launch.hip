@@ -114,11 +114,8 @@ struct Scratch {
     if (p) (void)hipFree(p);
   }
   int alloc(uint64_t bytes) {
-    if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
+    if (!device_alloc(&p, bytes ? bytes : 1))
       return fail(RFX_ENOMEM, "harmony: %llu bytes of scratch", static_cast<unsigned long long>(bytes));
-    }
     return RFX_OK;
   }
 };

@@ -322,11 +322,8 @@ struct Pool {
       *p = v.back();
       v.pop_back();
     } else {
-      if (hipMalloc(p, c) != hipSuccess) {
-        (void)hipGetLastError();
-        *p = nullptr;
+      if (!device_alloc(p, c))
         return fail(RFX_ENOMEM, "hir: allocating %llu bytes", static_cast<unsigned long long>(c));
-      }
       all.push_back(*p);
     }
     *cap = c;

@@ -74,6 +74,10 @@ inline bool valid_width(int b) {
 
 constexpr uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 
+// hipMalloc, after giving back the blocks that rfx_free keeps if there is no
+// room at first.  Null and false if there is none then; released by hipFree.
+bool device_alloc(void** ptr, uint64_t bytes);
+
 // Make sure ctx->ws holds `bytes` (synchronises the stream before growing).
 // Refused while graphs captured on the context are alive.
 int ensure_workspace(rfx_ctx* ctx, uint64_t bytes);

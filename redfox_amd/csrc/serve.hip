@@ -497,11 +497,9 @@ struct TempMem {
   template <class T>
   int take(uint64_t n, T** out) {
     void* q = nullptr;
-    if (hipMalloc(&q, (n ? n : 1) * sizeof(T)) != hipSuccess) {
-      (void)hipGetLastError();
+    if (!device_alloc(&q, (n ? n : 1) * sizeof(T)))
       return fail(RFX_ENOMEM, "serve: %llu bytes to measure a join",
                   static_cast<unsigned long long>(n * sizeof(T)));
-    }
     p.push_back(q);
     *out = static_cast<T*>(q);
     return RFX_OK;
@@ -592,12 +590,13 @@ int rfx_server_create(rfx_server** out, int device, int slots, uint64_t budget_b
   auto* s = new rfx_server;
   s->device = device;
   const uint64_t bytes = align_up(budget_bytes, 1u << 20);
-  if (hipMalloc(reinterpret_cast<void**>(&s->base), bytes) != hipSuccess) {
-    (void)hipGetLastError();
+  void* base = nullptr;
+  if (!device_alloc(&base, bytes)) {
     delete s;
     return fail(RFX_ENOMEM, "rfx_server_create: arena of %llu bytes",
                 static_cast<unsigned long long>(bytes));
   }
+  s->base = static_cast<char*>(base);
   s->arena.reset(bytes);
   s->slots.resize(slots);
   for (Slot& sl : s->slots) {
@@ -700,8 +699,11 @@ int rfx_server_run(rfx_server* s, rfx_request* reqs, uint64_t n, int mode, rfx_s
     reqs[i].admit_ns = reqs[i].done_ns = 0;
     reqs[i].status = RFX_OK;
   }
-  uint64_t* res = nullptr;
-  RFX_HIP(hipMalloc(reinterpret_cast<void**>(&res), (n ? n : 1) * kResWords * sizeof(uint64_t)));
+  void* res_mem = nullptr;
+  if (!device_alloc(&res_mem, (n ? n : 1) * kResWords * sizeof(uint64_t)))
+    return fail(RFX_EHIP, "rfx_server_run: no memory for the results of %llu requests",
+                static_cast<unsigned long long>(n));
+  uint64_t* res = static_cast<uint64_t*>(res_mem);
   s->arena.reset(s->arena.capacity());
   const int nslots = mode == RFX_SERVE_PLAIN ? 1 : static_cast<int>(s->slots.size());
   uint64_t next = 0, finished = 0, blocked = 0;

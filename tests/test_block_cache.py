@@ -1,6 +1,7 @@
 """The block cache behind rfx_malloc / rfx_free (csrc/block_cache.h), built
 with the host compiler over a runtime that hands out numbered addresses."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -99,7 +100,41 @@ CASES = {
   for (void* p : all) assert(put(c, d, p));
   assert(d.used == 512ull << 20);
 """,
+    "kept blocks make room for the library's own allocations": r"""
+  d.limit = 100 << 20;
+  void* a = get(c, 60 << 20);
+  void* in_use = get(c, 20 << 20);
+  assert(put(c, d, a) && d.live.count(a));
+  void* ws = nullptr;
+  assert(c.alloc(&ws, 70 << 20) && ws && !d.live.count(a) && d.live.count(in_use));
+  assert(!put(c, d, a));              // given back: the runtime refuses it
+  Fake{&d}.release(ws);
+  void* b = nullptr;
+  assert(!c.alloc(&b, 90 << 20));     // in use: no room, nothing kept to give back
+  assert(put(c, d, in_use) && d.live.count(in_use));
+  d.capturing = true;                 // no waiting for the device then
+  assert(!c.alloc(&b, 90 << 20) && d.live.count(in_use));
+  d.capturing = false;
+  assert(c.alloc(&b, 90 << 20));
+""",
+    "and for rfx_malloc": r"""
+  d.limit = 100 << 20;
+  void* a = get(c, 60 << 20);
+  assert(put(c, d, a));
+  void* b = get(c, 63 << 20);
+  assert(b && !d.live.count(a) && put(c, d, b));
+  void* e = get(c, (64 << 20) - 5);   // its rounded size fits once the kept block is gone
+  assert(e && d.live.at(e) >= (64 << 20) - 5);
+""",
 }
+
+
+def test_every_device_allocation_can_reclaim_kept_blocks():
+    """hipMalloc has one caller: the runtime under the cache."""
+    csrc = os.path.join(ROOT, "redfox_amd", "csrc")
+    calls = [(f, line.strip()) for f in sorted(os.listdir(csrc)) if f.endswith((".hip", ".cpp", ".h"))
+             for line in open(os.path.join(csrc, f)) if re.search(r"hipMalloc(Async|Managed)?\s*\((?!%)", line)]
+    assert calls == [("context.hip", "if (hipMalloc(p, bytes) == hipSuccess) return true;")]
 
 
 def run(tmp_path, body):
