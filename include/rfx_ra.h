@@ -101,8 +101,9 @@ int rfx_device_count(int* count);
 int rfx_set_device(int device);
 /* rfx_free waits for the device, as hipFree does, and may keep the block
  * (up to 64 MiB each, 512 MiB in all) for a later rfx_malloc; kept blocks go
- * back to the runtime when an allocation fails and when a context is
- * destroyed. */
+ * back to the runtime when an allocation of the library finds no room and
+ * when the last context is destroyed.  A second rfx_free of a block is
+ * refused. */
 int rfx_malloc(void** ptr, uint64_t bytes);
 int rfx_free(void* ptr);
 int rfx_memcpy_htod(void* dst, const void* src, uint64_t bytes);
@@ -110,6 +111,7 @@ int rfx_memcpy_dtoh(void* dst, const void* src, uint64_t bytes);
 int rfx_memcpy_dtod(void* dst, const void* src, uint64_t bytes);
 int rfx_memset(void* dst, int value, uint64_t bytes);
 int rfx_device_synchronize(void);
+/* Free bytes include the blocks that rfx_free keeps. */
 int rfx_mem_info(uint64_t* free_bytes, uint64_t* total_bytes);
 
 /* Per-launch timing: while enabled, every kernel launch of the operators

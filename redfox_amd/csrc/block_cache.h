@@ -7,7 +7,7 @@
 // queued work of any stream or thread can still touch it, so it may be
 // handed to any of them.  Blocks of up to kKeepBlock bytes, kKeepTotal in
 // all; they go back to the runtime when an allocation fails (any of the
-// library's: alloc) and when a context is destroyed.  Other pointers, other devices' blocks and frees
+// library's: alloc) and when the last context is destroyed.  Other pointers, other devices' blocks and frees
 // while a graph is being captured (no waiting then) go straight to the
 // runtime.
 //
@@ -98,6 +98,30 @@ class BlockCache {
     return kKept;
   }
 
+  // Contexts come and go while others work (a server makes one per slot), so
+  // the blocks stay until none is left: giving them back waits for the device
+  // block by block.
+  void context_made() {
+    std::lock_guard<std::mutex> hold(mu_);
+    ++contexts_;
+  }
+  void context_gone() {
+    {
+      std::lock_guard<std::mutex> hold(mu_);
+      if (--contexts_) return;
+    }
+    drop();
+  }
+
+  // Bytes kept on a device.
+  uint64_t kept(int dev) {
+    std::lock_guard<std::mutex> hold(mu_);
+    uint64_t sum = 0;
+    for (auto& f : free_)
+      if (f.first.first == dev) sum += f.first.second * f.second.size();
+    return sum;
+  }
+
   // Gives every kept block back to the runtime; false if there was none.
   bool drop() {
     std::vector<void*> all;
@@ -135,6 +159,7 @@ class BlockCache {
   std::map<std::pair<int, uint64_t>, std::vector<void*>> free_;  // by device and size
   std::map<void*, Block> blocks_;                                // handed out or kept
   uint64_t kept_ = 0;
+  int64_t contexts_ = 0;
 };
 
 }  // namespace rfx

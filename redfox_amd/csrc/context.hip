@@ -295,6 +295,7 @@ int rfx_ctx_create(rfx_ctx** out, int device, void* stream) {
           hipSuccess &&
       cus > 0)
     c->device_cus = cus;
+  g_blocks.context_made();
   *out = c;
   return RFX_OK;
 }
@@ -313,7 +314,7 @@ int rfx_ctx_destroy(rfx_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipFree(ctx->cells);
   }
-  g_blocks.drop();
+  g_blocks.context_gone();
   delete ctx;
   return RFX_OK;
 }
@@ -486,8 +487,10 @@ int rfx_device_synchronize(void) {
 }
 int rfx_mem_info(uint64_t* free_bytes, uint64_t* total_bytes) {
   size_t f = 0, t = 0;
+  int dev = 0;
   RFX_HIP(hipMemGetInfo(&f, &t));
-  if (free_bytes) *free_bytes = f;
+  RFX_HIP(hipGetDevice(&dev));
+  if (free_bytes) *free_bytes = f + g_blocks.kept(dev);  // an allocation may have those too
   if (total_bytes) *total_bytes = t;
   return RFX_OK;
 }

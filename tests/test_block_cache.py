@@ -126,6 +126,23 @@ CASES = {
   void* e = get(c, (64 << 20) - 5);   // its rounded size fits once the kept block is gone
   assert(e && d.live.at(e) >= (64 << 20) - 5);
 """,
+    "kept blocks outlive a context and go back with the last one": r"""
+  c.context_made(); c.context_made();
+  void* a = get(c, 1000);
+  assert(put(c, d, a));
+  c.context_gone();
+  assert(d.live.count(a) && get(c, 1000) == a && put(c, d, a));
+  c.context_gone();
+  assert(!d.live.count(a) && d.used == 0);
+""",
+    "kept bytes are counted by device": r"""
+  void* a = get(c, 1000); void* b = get(c, 3 << 20);
+  assert(c.kept(0) == 0 && put(c, d, a) && put(c, d, b));
+  d.dev = 1;
+  void* e = get(c, 2000);
+  assert(put(c, d, e));
+  assert(c.kept(0) + c.kept(1) == d.used && c.kept(1) == d.live.at(e));
+""",
 }
 
 

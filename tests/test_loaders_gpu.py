@@ -193,6 +193,21 @@ def test_second_free_is_refused(rf, size):
         assert lib.rfx_free(p) == 0
 
 
+
+def test_freed_memory_is_free(rf):
+    """rfx_mem_info after rfx_free: what was freed counts, kept or not."""
+    def free():
+        f, t = ctypes.c_uint64(), ctypes.c_uint64()
+        assert rf.lib().rfx_mem_info(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    bufs = [rf.DeviceBuffer(48 << 20) for _ in range(6)]
+    held = free()
+    for b in bufs:
+        b.close()
+    assert free() >= held + 6 * (48 << 20)
+
+
 # Fields that the word-wise conversion takes and those it leaves to the byte
 # loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
 # 3 digits after them, letters inside; dates of other shapes; rows short of
