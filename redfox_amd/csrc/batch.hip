@@ -141,13 +141,29 @@ __global__ __launch_bounds__(kCopyNT) void k_copy(const uint4* __restrict__ src,
     reinterpret_cast<uint8_t*>(dst)[tail] = reinterpret_cast<const uint8_t*>(src)[tail];
 }
 
-bool own_memory(rfx_ctx* ctx, const void* p) {
+// The device whose memory holds p, or -1.
+int device_of(const void* p) {
   hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+  if (hipPointerGetAttributes(&a, p) == hipSuccess)
+    return a.type == hipMemoryTypeDevice ? a.device : -1;
+  (void)hipGetLastError();
+  return -1;
+}
+
+// Which copy takes [p, p + bytes): ours if it lies within one allocation of
+// the context's device, none if it begins in an allocation and ends in no
+// memory, else the runtime's.
+enum class Copy { kOurs, kRuntime, kNone };
+Copy copy_of(rfx_ctx* ctx, const void* p, uint64_t bytes) {
+  if (device_of(p) != ctx->device) return Copy::kRuntime;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return Copy::kRuntime;
   }
-  return a.type == hipMemoryTypeDevice && a.device == ctx->device;
+  if (range_within(p, bytes, base, size)) return Copy::kOurs;
+  return device_of(static_cast<const char*>(p) + bytes - 1) < 0 ? Copy::kNone : Copy::kRuntime;
 }
 
 }  // namespace
@@ -227,12 +243,20 @@ int rfx_graph_destroy(void* graph_exec) {
 int rfx_copy(rfx_ctx* ctx, void* dst, const void* src, uint64_t bytes) {
   if (!ctx || (bytes && (!dst || !src))) return fail(RFX_EINVAL, "rfx_copy: null argument");
   if (!bytes) return RFX_OK;
-  // A large copy between this device's own allocations; the runtime's copy
-  // takes any other pointers (and small copies, which are all launch).
-  if (bytes >= kCopyMin && reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(src) % 16 == 0 && own_memory(ctx, dst) && own_memory(ctx, src)) {
+  // A large copy between aligned ranges of this device's own allocations that
+  // do not overlap; the runtime's copy takes any other pointers (and small
+  // copies, which are all launch).
+  const uintptr_t d = reinterpret_cast<uintptr_t>(dst), s = reinterpret_cast<uintptr_t>(src);
+  int dev = -1;
+  if (bytes >= kCopyMin && d % 16 == 0 && s % 16 == 0 && hipGetDevice(&dev) == hipSuccess &&
+      dev == ctx->device) {
+    const Copy to = copy_of(ctx, dst, bytes), from = copy_of(ctx, src, bytes);
+    if (to == Copy::kNone || from == Copy::kNone)
+      return fail(RFX_EHIP, "rfx_copy: %llu bytes leave the allocation they begin in",
+                  static_cast<unsigned long long>(bytes));
     const uint64_t blocks = (bytes + kCopyBlock - 1) / kCopyBlock;
-    if (blocks <= 0x7FFFFFFFull) {
+    const bool apart = (d > s ? d - s : s - d) >= bytes;
+    if (apart && to == Copy::kOurs && from == Copy::kOurs && blocks <= 0x7FFFFFFFull) {
       k_copy<<<static_cast<uint32_t>(blocks), kCopyNT, 0, ctx->stream>>>(
           static_cast<const uint4*>(src), static_cast<uint4*>(dst), bytes);
       RFX_LAUNCHED();

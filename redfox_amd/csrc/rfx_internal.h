@@ -78,6 +78,12 @@ constexpr uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a
 // room at first.  Null and false if there is none then; released by hipFree.
 bool device_alloc(void** ptr, uint64_t bytes);
 
+// [p, p + bytes) within [base, base + size).
+inline bool range_within(const void* p, uint64_t bytes, const void* base, uint64_t size) {
+  const uint64_t off = reinterpret_cast<uintptr_t>(p) - reinterpret_cast<uintptr_t>(base);
+  return off <= size && bytes <= size - off;
+}
+
 // Make sure ctx->ws holds `bytes` (synchronises the stream before growing).
 // Refused while graphs captured on the context are alive.
 int ensure_workspace(rfx_ctx* ctx, uint64_t bytes);

@@ -208,6 +208,32 @@ def test_freed_memory_is_free(rf):
     assert free() >= held + 6 * (48 << 20)
 
 
+
+@pytest.mark.parametrize("short", ["dst", "src"])
+def test_copy_past_an_allocation_is_refused(rf, ctx, short):
+    """The library's own copy kernel is not started on a range that leaves
+    its allocation (the runtime's copy refused it too).  The range ends far
+    beyond any memory, so the host refuses it whatever lies in between."""
+    big, small = rf.DeviceBuffer(160 << 20), rf.DeviceBuffer(70 << 20)
+    src, dst = (big, small) if short == "dst" else (small, big)
+    with pytest.raises(rf.RfxError):
+        ctx.copy(dst, src, 1 << 45)
+    ctx.copy(dst, src, 70 << 20)  # whole allocations are fine
+    ctx.synchronize()
+
+
+def test_copies_within_one_buffer(rf, ctx):
+    """Both ranges in one allocation, side by side up to its last byte."""
+    half = (80 << 20) + 16
+    buf = rf.DeviceBuffer(2 * half)
+    ctx.gen_u32(buf, half // 2, 9)
+    want = buf.download(np.uint8, half)
+    ctx.copy(buf, buf, half, dst_off=half, src_off=0)
+    ctx.synchronize()
+    got = buf.download(np.uint8, 2 * half)
+    assert np.array_equal(got[:half], want) and np.array_equal(got[half:], want)
+
+
 # Fields that the word-wise conversion takes and those it leaves to the byte
 # loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
 # 3 digits after them, letters inside; dates of other shapes; rows short of
