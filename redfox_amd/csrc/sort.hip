@@ -248,10 +248,11 @@ struct TileQueue {
 };
 
 // Rows of status words of one pass: the tiles, then the groups of a sort
-// whose tiles all run at once.
+// whose tiles all run at once (at most kGroupedTiles; a larger sort has rows
+// for as many, so that more tiles never need fewer rows).
 constexpr uint64_t kGroupedTiles = 2048;
 __host__ __device__ constexpr uint64_t status_rows(uint64_t tiles) {
-  return tiles + (tiles <= kGroupedTiles ? (tiles + kGroup - 1) / kGroup : 0);
+  return tiles + ((tiles < kGroupedTiles ? tiles : kGroupedTiles) + kGroup - 1) / kGroup;
 }
 
 struct SortLayout {
@@ -866,7 +867,13 @@ template <int KB, int VB>
 uint64_t sort_ws_bytes(uint64_t n, int key_bits) {
   using Tn = SortTune<KB, VB, 8>;
   const uint64_t tile = static_cast<uint64_t>(Tn::NT) * Tn::IPT;
-  if (n > kCountMask) return sort_ws_tile(n, KB, VB, key_bits, tile, 8, true);
+  if (n > kCountMask) {
+    // 64-bit words for larger tiles: no less than the most rows with 32-bit
+    // words and the smallest tile take.
+    const uint64_t wide = sort_ws_tile(n, KB, VB, key_bits, tile, 8, true);
+    const uint64_t narrow = sort_ws_bytes<KB, VB>(kCountMask, key_bits);
+    return wide > narrow ? wide : narrow;
+  }
   constexpr uint64_t kMinTile = kTuneNT * kSortMinIPT;
   uint64_t ws = sort_ws_tile(n, KB, VB, key_bits,
                              kSortTunable<KB, VB> && kMinTile < tile ? kMinTile : tile, 8);
