@@ -80,10 +80,15 @@ void* rfx_ctx_stream(rfx_ctx* ctx);
 int rfx_ctx_reserve(rfx_ctx* ctx, uint64_t bytes);
 uint64_t rfx_ctx_workspace_bytes(rfx_ctx* ctx);
 /* Tile shapes of the context's operators, for an autotuner: "sort.ipt"
- * (keys per thread of the onesweep tile: 8, 12 or 16, for 4/8-byte keys
- * with 0/4/8-byte values), "sort.digit" (radix digit bits, 8, 9 or 10, for
- * the same shapes; 0 chooses from key_bits: 9 for 17-18 bits, 10 for
- * 19-20, 6 for 21-24, 7 for 25-28, else 8), "join.fb_tile" and "join.ex_tile" (2048 or 4096 merged
+ * (keys per thread of the onesweep tile, of 512 threads: 8, 12 or 16, for
+ * 4/8-byte keys with 0/4/8-byte values and 8-bit digits; of these 12 also for
+ * 9 and 10-bit digits; 0 chooses 8 to 32 keys of 512 or 1024 threads by the
+ * widths and the rows), "sort.digit" (radix digit bits, 6 to 10, for the same
+ * shapes; 0 chooses from key_bits: 9 for 17-18 bits, 10 for 19-20, 6 for
+ * 21-24, 7 for 25-28, else 8; with sort.ipt set, 8 for 21-28; digits of 6 and
+ * 7 bits take the tile that sort.ipt 0 chooses); a context with either knob
+ * set also sorts up to 8192 rows by tiles instead of in one block,
+ * "join.fb_tile" and "join.ex_tile" (2048 or 4096 merged
  * items per find_bounds / expansion tile), "select.vt" (rows per thread of
  * the select pass: 8, 16, 24 or 32), "mapfilter.mode" (1: run programs
  * compiled for their types only, 2: interpret them only; the default 0

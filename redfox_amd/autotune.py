@@ -24,7 +24,7 @@ from . import rfx as R
 # knob -> candidates, the built-in default (0) first
 KNOBS: Dict[str, Tuple[int, ...]] = {
     "sort.ipt": (0, 8, 12, 16),
-    "sort.digit": (0, 8, 9, 10),
+    "sort.digit": (0, 6, 7, 8, 9, 10),
     "join.fb_tile": (0, 2048),
     "join.ex_tile": (0, 2048),
     "select.vt": (0, 8, 16, 24, 32),

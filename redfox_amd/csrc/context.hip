@@ -345,9 +345,9 @@ static int* tune_field(rfx_ctx* ctx, const char* knob, const int** allowed, int*
     return &ctx->tune_sort_ipt;
   }
   if (!std::strcmp(knob, "sort.digit")) {
-    static const int digits[] = {0, 8, 9, 10};
+    static const int digits[] = {0, 6, 7, 8, 9, 10};
     *allowed = digits;
-    *nallowed = 4;
+    *nallowed = 6;
     return &ctx->tune_sort_digit;
   }
   if (!std::strcmp(knob, "sort.status")) {

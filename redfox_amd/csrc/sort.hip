@@ -990,9 +990,12 @@ int sort_tuned(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
     return RFX_OK;
   }
   if constexpr (kSortTunable<KB, VB>) {
-    // Knob value 0 takes the digit width chosen for key_bits.
-    const int digit = ctx->tune_sort_digit ? ctx->tune_sort_digit : auto_digit(key_bits);
+    // Knob value 0 takes the digit width chosen for key_bits; tiles of a set
+    // number of keys exist for 8 bits and wider.
     const int ipt = ctx->tune_sort_ipt;
+    const int digit = ctx->tune_sort_digit            ? ctx->tune_sort_digit
+                      : ipt && auto_digit(key_bits) < 8 ? 8
+                                                        : auto_digit(key_bits);
     if (digit == 6) return sort_digits<KB, VB, 6>(ctx, keys, vals, n, key_bits);
     if (digit == 7) return sort_digits<KB, VB, 7>(ctx, keys, vals, n, key_bits);
     if (digit == 9)

@@ -265,3 +265,27 @@ def test_one_block_sorts_match_oracle(rf, ctx, orc, kb, vb, bits, n):
     assert np.array_equal(gk, ok)
     if vb:
         assert np.array_equal(gv, ov)
+
+
+@pytest.mark.parametrize("digit,ipt,bits,passes", [
+    (0, 0, 22, 4), (0, 8, 22, 3), (0, 12, 27, 4), (0, 16, 24, 3), (8, 0, 22, 3), (6, 0, 32, 6), (7, 0, 32, 5),
+    (6, 8, 22, 4), (0, 12, 20, 2)])
+def test_sort_knobs_are_honoured(rf, ctx, digit, ipt, bits, passes):
+    """A set sort.ipt takes 8-bit digits where the default would be 6 or 7
+    bits (the number of passes tells), and 6 and 7 bits can be asked for."""
+    n = 200_003
+    keys = make(4, n, 1200 + bits)
+    vals = np.arange(n, dtype=np.uint32)
+    try:
+        ctx.tune("sort.digit", digit)
+        ctx.tune("sort.ipt", ipt)
+        ctx.profile(True)
+        gk, gv = run_sort(rf, ctx, keys, vals, 4, bits, 4)
+        launches, _ = ctx.profile_read("sort.onesweep")
+    finally:
+        ctx.profile(False)
+        ctx.tune("sort.digit", 0)
+        ctx.tune("sort.ipt", 0)
+    order = np.argsort(keys & np.uint32((1 << bits) - 1), kind="stable")
+    assert np.array_equal(gk, keys[order]) and np.array_equal(gv, vals[order])
+    assert launches == passes
