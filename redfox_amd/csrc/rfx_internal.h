@@ -50,13 +50,16 @@ extern std::atomic<int> g_capturing;
 // Record an error message for rfx_last_error() and return `code`.
 int fail(int code, const char* fmt, ...);
 
-// Check a HIP call; on failure record it and return RFX_EHIP.
-#define RFX_HIP(call)                                                   \
-  do {                                                                  \
-    hipError_t rfx_e_ = (call);                                         \
-    if (rfx_e_ != hipSuccess)                                           \
-      return ::rfx::fail(RFX_EHIP, "%s failed: %s (%s:%d)", #call,      \
+// Check a HIP call; on failure record it and return RFX_EHIP.  The runtime's
+// own record is cleared, or the thread's next launch would report it again.
+#define RFX_HIP(call)                                                    \
+  do {                                                                   \
+    hipError_t rfx_e_ = (call);                                          \
+    if (rfx_e_ != hipSuccess) {                                          \
+      (void)hipGetLastError();                                           \
+      return ::rfx::fail(RFX_EHIP, "%s failed: %s (%s:%d)", #call,       \
                          hipGetErrorString(rfx_e_), __FILE__, __LINE__); \
+    }                                                                    \
   } while (0)
 
 #define RFX_TRY(expr)            \

@@ -234,6 +234,19 @@ def test_copies_within_one_buffer(rf, ctx):
     assert np.array_equal(got[:half], want) and np.array_equal(got[half:], want)
 
 
+
+def test_a_refused_call_leaves_the_next_launch_alone(rf, ctx):
+    """An error of the runtime belongs to the call that met it: the next
+    operator of the thread, which checks its launch, does not report it."""
+    p = ctypes.c_void_p()
+    assert rf.lib().rfx_malloc(ctypes.byref(p), (64 << 20) + 1) == 0
+    assert rf.lib().rfx_free(p.value) == 0
+    assert rf.lib().rfx_free(p.value) != 0
+    buf = rf.DeviceBuffer(4096)
+    ctx.gen_u32(buf, 1024, 5)
+    assert np.array_equal(buf.download(np.uint32, 1024), datagen.u32(5, 1024))
+
+
 # Fields that the word-wise conversion takes and those it leaves to the byte
 # loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
 # 3 digits after them, letters inside; dates of other shapes; rows short of
