@@ -247,6 +247,64 @@ def test_a_refused_call_leaves_the_next_launch_alone(rf, ctx):
     assert np.array_equal(buf.download(np.uint32, 1024), datagen.u32(5, 1024))
 
 
+# Row ends where a text's first and last 16-byte words are cut: every
+# alignment of the first byte, lengths about whole words, one tile of 64 KB
+# and two, with newlines at both ends of the text and neighbours outside it.
+@pytest.mark.parametrize("size", [1, 15, 16, 17, 40, 65_519, 65_520, 65_521, 65_535, 65_536, 65_537, 131_075])
+def test_row_ends_at_any_alignment(rf, ctx, size):
+    rng = np.random.default_rng(size)
+    for off in range(16):
+        body = rng.choice(np.frombuffer(b"0123456789\n", np.uint8), size, p=[0.08] * 10 + [0.2])
+        if off % 3 == 0:
+            body[0] = 10
+        if off % 2 == 0:
+            body[-1] = 10
+        text = body.tobytes()
+        host = np.full(off + size + 64, 10, np.uint8)  # newlines all around
+        host[off:off + size] = body
+        buf = rf.DeviceBuffer.from_numpy(host)
+
+        class At:
+            ptr = buf.ptr + off
+        want, _ = oracle.parse_tbl(text, ["i64"])
+        for cap in (max(1, len(want[0])), 7):
+            out, cells = rf.DeviceBuffer(8 * cap), rf.DeviceBuffer(16)
+            types = (ctypes.c_int * 1)(loaders.TBL["i64"])
+            ptrs = (ctypes.c_void_p * 1)(out.ptr)
+            assert rf.lib().rfx_tbl_parse(ctx.handle, At.ptr, size, b"|", types, 1, ptrs, cap,
+                                          cells.ptr, cells.ptr + 8) == 0
+            assert cells.download(np.uint64, 2)[0] == len(want[0]), off
+            m = min(cap, len(want[0]))
+            assert np.array_equal(out.download(np.int64, m), want[0][:m]), off
+
+
+def test_a_cut_tile_costs_about_a_whole_one(rf, ctx):
+    """Row ends of a text one byte short of a tile (4.5 times a whole tile's
+    time where the cut tile was read byte by byte), and of an unaligned one."""
+    size = 65_536
+    buf = rf.DeviceBuffer.from_numpy(np.frombuffer((b"12345|abcdefghij|0.25\n" * 4000)[:size + 16], np.uint8))
+    out, cells = rf.DeviceBuffer(8 * size), rf.DeviceBuffer(16)
+    types = (ctypes.c_int * 1)(loaders.TBL["i64"])
+    ptrs = (ctypes.c_void_p * 1)(out.ptr)
+
+    def row_ends_ms(off, n):
+        best = 1e9
+        for _ in range(5):
+            ctx.profile(True)
+            for _ in range(20):
+                assert rf.lib().rfx_tbl_parse(ctx.handle, buf.ptr + off, n, b"|", types, 1, ptrs, size,
+                                              cells.ptr, cells.ptr + 8) == 0
+            launches, ms = ctx.profile_read("tbl.rows")
+            ctx.profile(False)
+            assert launches == 20
+            best = min(best, ms / launches)
+        return best
+
+    whole = row_ends_ms(0, size)
+    assert row_ends_ms(0, size - 1) < 3 * whole
+    assert row_ends_ms(3, size - 16) < 3 * whole
+
+
 # Fields that the word-wise conversion takes and those it leaves to the byte
 # loop: lengths about 8 digits, signs, spaces, points first, last, twice, 0 to
 # 3 digits after them, letters inside; dates of other shapes; rows short of
