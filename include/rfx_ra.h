@@ -235,10 +235,11 @@ int rfx_join_find_bounds_string(rfx_ctx* ctx, int32_t* lower_bound, int32_t* lef
                                 uint64_t* total, const uint64_t* left, uint64_t nl,
                                 const uint64_t* right, uint64_t nr);
 /* Sort n string addresses in place into compare_string2's order, stably
- * (equal strings keep their order); scratch holds n + 1 u64.  No reference
- * counterpart takes unsorted string columns: the reference's string keys
- * arrive sorted.  Synchronises the stream once (the longest string sets
- * the number of passes). */
+ * (equal strings keep their order); scratch holds n + 1 u64 (n are used).
+ * No reference counterpart takes unsorted string columns: the reference's
+ * string keys arrive sorted.  Synchronises the stream once: the bits in which
+ * the strings differ within their first 256 bytes, and the longest string
+ * beyond, set the sort keys and the number of passes. */
 int rfx_sort_strings(rfx_ctx* ctx, uint64_t* addresses, uint64_t* scratch, uint64_t n);
 /* The same order as a permutation: rows (n u32 row numbers below n, e.g.
  * 0..n-1) is sorted stably by the string of each row, addresses[row]

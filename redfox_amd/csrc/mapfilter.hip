@@ -68,9 +68,7 @@ __global__ __launch_bounds__(kMNT) void k_mapfilter(MfIn in, uint64_t n, rfx_mf_
                                                     uint64_t* __restrict__ status,
                                                     uint32_t* __restrict__ ticket) {
   mapfilter_tile<1, 1>(
-      [&](uint64_t r) {
-        return prog.n_filter == 0 || run_ops(prog, 0, prog.n_filter, in, out, r, 0) != 0;
-      },
+      [&](uint64_t r) { return run_ops(prog, 0, prog.n_filter, in, out, r, 0) != 0; },
       [](uint64_t) { return Empty{}; },
       [&](uint64_t r, uint64_t pos, Empty) {
         run_ops(prog, prog.n_filter, prog.n_ops, in, out, r, pos);

@@ -28,10 +28,12 @@ namespace {
 #endif
 constexpr int kFNT = RFX_SEL_NT;
 constexpr int kFNW = kFNT / kWave;
-// Rows per thread by default, from the autotuner's sweep over the same
-// 2 GiB of tuples with half kept (ms for 8 / 16 / 24 / 32 rows): 16-byte
-// tuples 0.74 / 0.68 / 0.63 / 0.74, 8-byte 1.06 / 0.84 / 0.72 / 0.78,
-// 4-byte 1.71 / 1.24 / 1.05 / 0.96.  The select.vt knob picks 8, 16, 24 or
+// Rows per thread by default (u32 field below the middle, half kept; us for
+// 8 / 16 / 24 / 32 rows): 2^27 rows of 16 bytes 727 / 623 / 590 / 649, of 8
+// bytes 515 / 391 / 356 / 349, of 4 bytes 436 / 279 / 236 / 229; 2^20 rows 12.1
+// / 11.6 / 13.0 / 14.5, 11.0 / 10.4 / 11.5 / 12.5 and 10.8 / 9.2 / 10.2 / 10.8.
+// 8-byte tuples lie between: 32 rows gain 2 to 4% from 2^22 rows on (nothing
+// at 2^26) and lose 9% at 2^20, so 24.  The select.vt knob picks 8, 16, 24 or
 // 32 instead.
 template <class K>
 constexpr int kFVT = sizeof(K) >= 16 ? RFX_SEL_VT16 : sizeof(K) == 8 ? 24 : 32;
