@@ -255,6 +255,19 @@ __host__ __device__ constexpr uint64_t status_rows(uint64_t tiles) {
   return tiles + ((tiles < kGroupedTiles ? tiles : kGroupedTiles) + kGroup - 1) / kGroup;
 }
 
+// Tiles per resident block from which the queues pay.  Their chunks wait for
+// one another in the look-back, so with few of them, or where a tile writes
+// little, one ticket is faster (whole sorts, ms by queues / by one ticket):
+// (4, 4) 14 M rows 0.306 / 0.274, 30 M 0.573 / 0.620; (8, 4) 14 M 0.805 / 0.755,
+// 20 M 1.093 / 1.168; (4, 1) 30 M 0.500 / 0.483, 64 M 0.981 / 0.993; (16, 0) 14 M
+// 2.06 / 1.97, 30 M 4.16 / 4.65; (8, 0) 64 M 2.58 / 2.51, 134 M 5.06 / 5.23;
+// (4, 0) 64 M 0.825 / 0.764, 268 M 2.97 / 2.89.
+template <int KB, int VB>
+constexpr uint64_t kQueueFrom = VB >= 4             ? 4
+                                : VB > 0 || KB == 16 ? 8
+                                : KB == 8            ? 24
+                                                     : 64;
+
 struct SortLayout {
   uint32_t* hist;    // [P][bins]
   uint32_t* base;    // [P][bins] exclusive global digit offsets
@@ -939,7 +952,8 @@ int sort_impl(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
   // one request at a time, where nothing waits: 993 and 982.
   const bool shared = ctx->ws_borrowed;
   const uint32_t grid = static_cast<uint32_t>(tiles < slots || shared ? tiles : slots);
-  const uint32_t first = tiles > 2 * slots && !shared ? (grid + kQueues - 1) / kQueues : 0;
+  const uint32_t first =
+      tiles > kQueueFrom<KB, VB> * slots && !shared ? (grid + kQueues - 1) / kQueues : 0;
   for (int p = 0; p < passes; ++p) {
     RFX_PROF(ctx, "sort.onesweep");
     k_onesweep<KB, VB, NT, IPT, DB, LBW, S><<<grid, NT, 0, ctx->stream>>>(

@@ -227,8 +227,8 @@ def test_more_than_2p30_rows_properties(rf, ctx):
     assert seen.all()
 
 
-# Past 2 x 256 CUs x 2 blocks of the largest tile, where tiles are handed out
-# by the XCDs' queues; the last size of the small tiles and the next; group
+# Past 2 x 256 CUs x 2 blocks of the largest tile, where blocks that stay take
+# their tiles from one ticket; the last size of the small tiles and the next; group
 # and tile edges of the small tiles; even and odd numbers of 6 and 7 bit
 # digits (a skipped pass included).
 @pytest.mark.parametrize("kb,vb,bits,n", [
@@ -244,6 +244,27 @@ def test_tile_queues_and_small_tiles_match_numpy(rf, ctx, kb, vb, bits, n):
     vals = make(vb, n, 1001) if vb else None
     gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
     order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gk, keys[order])
+    if vb:
+        assert np.array_equal(gv, vals[order])
+
+
+# The first sizes past which tiles come from the queues (4, 8, 24 and 64 tiles
+# for each block that runs at once), and the last below, where one ticket
+# hands them out.
+@pytest.mark.parametrize("kb,vb,bits,n", [
+    (4, 4, 16, 2048 * 12_288), (4, 4, 16, 2048 * 12_288 + 1), (8, 4, 11, 2048 * 7168 + 5),
+    (8, 8, 16, 1024 * 12_288 + 5), (4, 8, 20, 1024 * 14_336 + 5), (8, 1, 16, 4096 * 7168 + 5),
+    (16, 0, 12, 4096 * 4096 + 5), (16, 4, 9, 2048 * 4096 + 5), (8, 0, 8, 12_288 * 7168 + 5)])
+def test_tile_queues_begin(rf, ctx, kb, vb, bits, n):
+    keys = make(kb, n, 1300 + bits)  # bits above key_bits vary and do not count
+    vals = make(vb, n, 1301) if vb else None
+    gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
+    low = keys[::2] if kb == 16 else keys  # word 0 is the low one
+    low = (low & low.dtype.type((1 << bits) - 1)).astype(np.uint16 if bits <= 16 else np.uint32)
+    order = np.argsort(low, kind="stable")
+    if kb == 16:
+        keys, gk = keys.reshape(-1, 2), gk.reshape(-1, 2)
     assert np.array_equal(gk, keys[order])
     if vb:
         assert np.array_equal(gv, vals[order])
