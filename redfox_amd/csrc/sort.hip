@@ -42,16 +42,22 @@ constexpr int kBinsOf = 1 << DB;
 // bits wide or keys and values are both 8 bytes, one block of 1024 (2^25
 // u32 keys of 20 bits with f64 values: 0.65 -> 0.57 ms; 2^26 u64 pairs
 // 3.97 -> 3.79 ms; u64 keys with u32 values 6.16 -> 7.1 ms, so not there).
+// 4-byte elements beside narrower ones take the tile of 24 as well past
+// mid_rows rows (2^28 rows, 16 -> 24: 2-byte keys with 4-byte values 2.48 ->
+// 2.08 ms, 4-byte keys with one-byte values 4.50 -> 3.82); at 1 M rows it is
+// too few tiles (0.073 against 0.083 ms).
 template <int KB, int VB, int DB>
 struct SortTune {
   static constexpr int kMax = KB > VB ? KB : VB;
   static constexpr bool kWide = kMax == 8 && (DB == 10 || (KB == 8 && VB == 8));
   static constexpr int NT = kWide ? 1024 : 512;
-  static constexpr int IPT = kMax >= 16             ? 8
-                             : kMax >= 8            ? (kWide && DB <= 8 ? 12 : 14)
-                             : KB == 4 && VB == 4   ? 24
-                             : KB == 4 && VB == 0   ? (DB <= 8 ? 32 : 24)
-                                                    : 16;
+  static constexpr int IPT = kMax >= 16                       ? 8
+                             : kMax >= 8                      ? (kWide && DB <= 8 ? 12 : 14)
+                             : KB >= 2 && VB > 0 && kMax == 4 ? 24
+                             : KB == 4 && VB == 0             ? (DB <= 8 ? 32 : 24)
+                                                              : 16;
+  // Up to mid_rows, in shapes that have no tile of kMidNT x kMidIPT.
+  static constexpr int kFewIPT = kMax >= 8 ? IPT : 16;
 };
 
 // Look-back window (status words per round trip): every extra word polled
@@ -69,6 +75,7 @@ constexpr int kMidNT = 1024;
 constexpr int kMidIPT = 4;
 constexpr uint64_t kMidTiles = 2;
 constexpr int kGroups = 0;  // as a look-back window
+constexpr uint64_t mid_rows(uint64_t cus, uint64_t tile) { return cus * kMidTiles * tile; }
 
 // Consecutive tiles that one XCD's queue takes at a time.  Fewer share fewer
 // lines; more keep the chunks after them waiting in their look-back (2^26
@@ -887,9 +894,8 @@ uint64_t sort_ws_bytes(uint64_t n, int key_bits) {
     const uint64_t narrow = sort_ws_bytes<KB, VB>(kCountMask, key_bits);
     return wide > narrow ? wide : narrow;
   }
-  constexpr uint64_t kMinTile = kTuneNT * kSortMinIPT;
-  uint64_t ws = sort_ws_tile(n, KB, VB, key_bits,
-                             kSortTunable<KB, VB> && kMinTile < tile ? kMinTile : tile, 8);
+  constexpr uint64_t kMinTile = kTuneNT * (kSortTunable<KB, VB> ? kSortMinIPT : Tn::kFewIPT);
+  uint64_t ws = sort_ws_tile(n, KB, VB, key_bits, kMinTile < tile ? kMinTile : tile, 8);
   if (kSortTunable<KB, VB> && auto_digit(key_bits) != 8) {
     const uint64_t w2 = sort_ws_tile(n, KB, VB, key_bits,
                                      auto_digit(key_bits) > 8 ? kTuneNT * 12ull : kMinTile,
@@ -979,8 +985,11 @@ int sort_digits(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) 
   using Tn = SortTune<KB, VB, DB>;
   constexpr int NT = DB > 8 ? kTuneNT : kMidNT, IPT = DB > 8 ? 12 : kMidIPT;
   if constexpr (kSortTunable<KB, VB>) {
-    if (n <= ctx->device_cus * kMidTiles * NT * IPT)
+    if (n <= mid_rows(ctx->device_cus, NT * IPT))
       return sort_impl<KB, VB, NT, IPT, DB, kGroups>(ctx, keys, vals, n, key_bits);
+  } else if constexpr (Tn::kFewIPT != Tn::IPT) {
+    if (n <= mid_rows(ctx->device_cus, kMidNT * kMidIPT))
+      return sort_impl<KB, VB, Tn::NT, Tn::kFewIPT, DB>(ctx, keys, vals, n, key_bits);
   }
   return sort_impl<KB, VB, Tn::NT, Tn::IPT, DB>(ctx, keys, vals, n, key_bits);
 }

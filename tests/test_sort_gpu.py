@@ -270,6 +270,19 @@ def test_tile_queues_begin(rf, ctx, kb, vb, bits, n):
         assert np.array_equal(gv, vals[order])
 
 
+# 4-byte elements beside narrower ones: the last size of the smaller tile, the
+# next one, and past the first queue sizes of both tiles.
+@pytest.mark.parametrize("kb,vb,bits", [(2, 4, 16), (4, 1, 16), (4, 2, 13)])
+@pytest.mark.parametrize("n", [8193, 2_097_152, 2_097_153, 2048 * 12_288 + 12_289, 4096 * 12_288 + 7])
+def test_narrow_columns_match_numpy(rf, ctx, kb, vb, bits, n):
+    keys = make(kb, n, 1400 + vb)
+    vals = make(vb, n, 1401)
+    gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
+    order = np.argsort((keys & DT[kb]((1 << bits) - 1)).astype(np.uint16), kind="stable")
+    assert np.array_equal(gk, keys[order])
+    assert np.array_equal(gv, vals[order])
+
+
 # Sorts of one block: steps and waves that are full, one row past, and the
 # last size (8192 rows, 4096 of 16-byte elements) with the next one; digits
 # that no key varies in, a narrow last digit, few distinct keys.
