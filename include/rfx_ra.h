@@ -84,8 +84,9 @@ uint64_t rfx_ctx_workspace_bytes(rfx_ctx* ctx);
  * 4/8-byte keys with 0/4/8-byte values and 8-bit digits; of these 12 also for
  * 9 and 10-bit digits; 0 chooses 8 to 32 keys of 512 or 1024 threads by the
  * widths and the rows), "sort.digit" (radix digit bits, 6 to 10, for the same
- * shapes; 0 chooses from key_bits: 9 for 17-18 bits, 10 for 19-20, 6 for
- * 21-24, 7 for 25-28, else 8; with sort.ipt set, 8 for 21-28; digits of 6 and
+ * shapes; 0 chooses from key_bits: 9 for 17-18 bits, 10 for 19-20, 7 for
+ * 25-28, 6 for 21-24 from 20 million rows with values and 64 million without
+ * on, else 8; with sort.ipt set, 8 for 21-28; digits of 6 and
  * 7 bits take the tile that sort.ipt 0 chooses); a context with either knob
  * set also sorts up to 8192 rows by tiles instead of in one block,
  * "join.fb_tile" and "join.ex_tile" (2048 or 4096 merged

@@ -3,10 +3,10 @@
 // digit that ranks a tile in registers/LDS, obtains its global digit offsets
 // by decoupled look-back and scatters through an LDS reorder buffer.  Digits
 // are 8 bits, or 6 to 10 where key_bits makes an even number of passes of
-// them (auto_digit): wider digits take fewer passes over the data at the
-// cost of more bins per tile (more ranking ballots and look-back words,
-// shorter runs per bin in the scatter), narrower ones save the copy back
-// after an odd number of passes.
+// them and they are faster (auto_digit): wider digits take fewer passes over
+// the data at the cost of more bins per tile (more ranking ballots and
+// look-back words, shorter runs per bin in the scatter), narrower ones save
+// the copy back after an odd number of passes.
 //
 // Replaces redfox::sort_pair / sort_key (b40cSort.cu:58-1021: b40c LSD
 // radix, 4-5 bit digits, upsweep + spine + downsweep per digit, pong
@@ -869,13 +869,17 @@ constexpr uint64_t kSortMaxRows = (1ull << 31) - 1;
 // pairs, 18 bits 3.36 ms against 5.04, 20 bits 4.04 against 4.90.  Wider
 // keys keep 8 bits (26 bits: 5.51 ms against 5.65 with 9; 32 bits: 5.56
 // against 6.29).
-// 21-24 bit keys take four passes of 6 bits instead of three of 8 and the
-// copy, 25-28 bit keys four of 7 bits: fewer bins per tile, so fewer lines
-// written in part.
-constexpr int auto_digit(int key_bits) {
+// Narrower digits have fewer bins per tile, so fewer lines written in part:
+// 25-28 bit keys take four passes of 7 bits, and 21-24 bit keys, from the
+// rows on where four passes of 6 bits are faster than three of 8 and the copy
+// (24 bits, ms by 6 / by 8 bits: u32 pairs 1.5 M rows 0.086 / 0.071, 16 M 0.293 /
+// 0.268, 24 M 0.433 / 0.441, 64 M 1.01 / 1.05; u32 keys alone 24 M 0.298 / 0.275,
+// 64 M 0.686 / 0.700).
+constexpr uint64_t six_bits_from(int val_bytes) { return val_bytes ? 20'000'000 : 64'000'000; }
+constexpr int auto_digit(int key_bits, uint64_t n, int val_bytes) {
   return key_bits >= 17 && key_bits <= 18   ? 9
          : key_bits >= 19 && key_bits <= 20 ? 10
-         : key_bits >= 21 && key_bits <= 24 ? 6
+         : key_bits >= 21 && key_bits <= 24 ? (n < six_bits_from(val_bytes) ? 8 : 6)
          : key_bits >= 25 && key_bits <= 28 ? 7
                                             : 8;
 }
@@ -896,10 +900,10 @@ uint64_t sort_ws_bytes(uint64_t n, int key_bits) {
   }
   constexpr uint64_t kMinTile = kTuneNT * (kSortTunable<KB, VB> ? kSortMinIPT : Tn::kFewIPT);
   uint64_t ws = sort_ws_tile(n, KB, VB, key_bits, kMinTile < tile ? kMinTile : tile, 8);
-  if (kSortTunable<KB, VB> && auto_digit(key_bits) != 8) {
-    const uint64_t w2 = sort_ws_tile(n, KB, VB, key_bits,
-                                     auto_digit(key_bits) > 8 ? kTuneNT * 12ull : kMinTile,
-                                     auto_digit(key_bits));
+  const int digit = auto_digit(key_bits, n, VB);
+  if (kSortTunable<KB, VB> && digit != 8) {
+    const uint64_t w2 =
+        sort_ws_tile(n, KB, VB, key_bits, digit > 8 ? kTuneNT * 12ull : kMinTile, digit);
     if (w2 > ws) ws = w2;
   }
   return ws;
@@ -1016,9 +1020,11 @@ int sort_tuned(rfx_ctx* ctx, void* keys, void* vals, uint64_t n, int key_bits) {
     // Knob value 0 takes the digit width chosen for key_bits; tiles of a set
     // number of keys exist for 8 bits and wider.
     const int ipt = ctx->tune_sort_ipt;
-    const int digit = ctx->tune_sort_digit            ? ctx->tune_sort_digit
-                      : ipt && auto_digit(key_bits) < 8 ? 8
-                                                        : auto_digit(key_bits);
+    int digit = ctx->tune_sort_digit;
+    if (!digit) {
+      digit = auto_digit(key_bits, n, VB);
+      if (ipt && digit < 8) digit = 8;
+    }
     if (digit == 6) return sort_digits<KB, VB, 6>(ctx, keys, vals, n, key_bits);
     if (digit == 7) return sort_digits<KB, VB, 7>(ctx, keys, vals, n, key_bits);
     if (digit == 9)

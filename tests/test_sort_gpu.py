@@ -229,8 +229,8 @@ def test_more_than_2p30_rows_properties(rf, ctx):
 
 # Past 2 x 256 CUs x 2 blocks of the largest tile, where blocks that stay take
 # their tiles from one ticket; the last size of the small tiles and the next; group
-# and tile edges of the small tiles; even and odd numbers of 6 and 7 bit
-# digits (a skipped pass included).
+# and tile edges of the small tiles; 7 bit digits with a skipped pass, odd
+# numbers of 8 bit digits.
 @pytest.mark.parametrize("kb,vb,bits,n", [
     (4, 4, 32, 12_582_912 + 12_289), (4, 0, 32, 16_777_216 + 1), (8, 4, 64, 7_340_032 + 77),
     (8, 8, 24, 6_291_456 + 12_287), (4, 8, 20, 7_340_032 + 14_337),
@@ -244,6 +244,26 @@ def test_tile_queues_and_small_tiles_match_numpy(rf, ctx, kb, vb, bits, n):
     vals = make(vb, n, 1001) if vb else None
     gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
     order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gk, keys[order])
+    if vb:
+        assert np.array_equal(gv, vals[order])
+
+
+# 6 and 7 bit digits, in even and odd numbers, on the small tiles (their group
+# edges and the last size) and on the large one.
+@pytest.mark.parametrize("digit", [6, 7])
+@pytest.mark.parametrize("kb,vb,bits,n", [
+    (4, 4, 23, 4_096 * 15), (4, 4, 21, 4_096 * 32 + 1), (8, 0, 22, 3_000_003), (8, 8, 24, 6_291_456 + 12_287),
+    (4, 8, 32, 2_097_152), (8, 4, 37, 100_003), (4, 0, 14, 2_097_153)])
+def test_narrow_digits_match_numpy(rf, ctx, digit, kb, vb, bits, n):
+    keys = make(kb, n, 1600 + bits)
+    vals = make(vb, n, 1601) if vb else None
+    try:
+        ctx.tune("sort.digit", digit)
+        gk, gv = run_sort(rf, ctx, keys, vals, kb, bits, vb)
+    finally:
+        ctx.tune("sort.digit", 0)
+    order = np.argsort(keys & DT[kb]((1 << bits) - 1), kind="stable")
     assert np.array_equal(gk, keys[order])
     if vb:
         assert np.array_equal(gv, vals[order])
@@ -302,11 +322,11 @@ def test_one_block_sorts_match_oracle(rf, ctx, orc, kb, vb, bits, n):
 
 
 @pytest.mark.parametrize("digit,ipt,bits,passes", [
-    (0, 0, 22, 4), (0, 8, 22, 3), (0, 12, 27, 4), (0, 16, 24, 3), (8, 0, 22, 3), (6, 0, 32, 6), (7, 0, 32, 5),
-    (6, 8, 22, 4), (0, 12, 20, 2)])
+    (0, 0, 26, 4), (0, 8, 22, 3), (0, 12, 27, 4), (0, 16, 24, 3), (8, 0, 22, 3), (6, 0, 32, 6), (7, 0, 32, 5),
+    (7, 0, 28, 4), (0, 8, 28, 4), (6, 8, 22, 4), (0, 12, 20, 2)])
 def test_sort_knobs_are_honoured(rf, ctx, digit, ipt, bits, passes):
-    """A set sort.ipt takes 8-bit digits where the default would be 6 or 7
-    bits (the number of passes tells), and 6 and 7 bits can be asked for."""
+    """6 and 7-bit digits can be asked for (the number of passes tells), and
+    every combination of the two knobs sorts."""
     n = 200_003
     keys = make(4, n, 1200 + bits)
     vals = np.arange(n, dtype=np.uint32)
@@ -322,4 +342,27 @@ def test_sort_knobs_are_honoured(rf, ctx, digit, ipt, bits, passes):
         ctx.tune("sort.ipt", 0)
     order = np.argsort(keys & np.uint32((1 << bits) - 1), kind="stable")
     assert np.array_equal(gk, keys[order]) and np.array_equal(gv, vals[order])
+    assert launches == passes
+
+
+@pytest.mark.parametrize("vb,n,ipt,passes", [
+    (4, 1_500_000, 0, 3), (4, 19_999_999, 0, 3), (4, 20_000_000, 0, 4), (4, 20_000_000, 16, 3),
+    (0, 20_000_000, 0, 3), (0, 64_000_000, 0, 4)])
+def test_six_bit_digits_where_they_pay(rf, ctx, vb, n, ipt, passes):
+    """23-bit keys: three passes of 8 bits below the rows where four of 6 bits
+    are faster, and with sort.ipt set, which has tiles for 8 bits only."""
+    keys = make(4, n, 1500) & np.uint32(0x7F00FF)  # 15 bits vary: a quick check on the host
+    vals = np.arange(n, dtype=np.uint32) if vb else None
+    try:
+        ctx.tune("sort.ipt", ipt)
+        ctx.profile(True)
+        gk, gv = run_sort(rf, ctx, keys, vals, 4, 23, vb)
+        launches, _ = ctx.profile_read("sort.onesweep")
+    finally:
+        ctx.profile(False)
+        ctx.tune("sort.ipt", 0)
+    order = np.argsort((keys & 0xFF | keys >> 8).astype(np.uint16), kind="stable")
+    assert np.array_equal(gk, keys[order])
+    if vb:
+        assert np.array_equal(gv, order.astype(np.uint32))
     assert launches == passes
