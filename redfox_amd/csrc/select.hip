@@ -33,10 +33,13 @@ constexpr int kFNW = kFNT / kWave;
 // bytes 515 / 391 / 356 / 349, of 4 bytes 436 / 279 / 236 / 229; 2^20 rows 12.1
 // / 11.6 / 13.0 / 14.5, 11.0 / 10.4 / 11.5 / 12.5 and 10.8 / 9.2 / 10.2 / 10.8.
 // 8-byte tuples lie between: 32 rows gain 2 to 4% from 2^22 rows on (nothing
-// at 2^26) and lose 9% at 2^20, so 24.  The select.vt knob picks 8, 16, 24 or
-// 32 instead.
+// at 2^26) and lose 9% at 2^20, so 24.  Up to kFewRows rows 8: a few tiles
+// are all latency, and theirs is the shortest (65,536 rows 6.6 us for 8 rows, 7.3
+// to 8.3 for 16, 9.0 to 10.0 for 24; 100 rows 9.0 with 24 or 32).  The select.vt
+// knob picks 8, 16, 24 or 32 instead.
 template <class K>
 constexpr int kFVT = sizeof(K) >= 16 ? RFX_SEL_VT16 : sizeof(K) == 8 ? 24 : 32;
+constexpr uint64_t kFewRows = 1ull << 16;
 
 // The comparisons of Comparisons.h:115-300.  Every integer one keeps an
 // interval of the field's values, or all but one: with the field's sign bit
@@ -319,7 +322,7 @@ int select_vt(rfx_ctx* ctx, void* out, uint64_t* n_out, const void* in, uint64_t
   return RFX_OK;
 }
 
-// Rows per thread: the built-in kFVT<K>, or the context's select.vt knob.
+// Rows per thread: by the rows (8, kFVT<K>), or the context's select.vt knob.
 template <class K>
 int select_impl(rfx_ctx* ctx, void* out, uint64_t* n_out, const void* in, uint64_t n, Pred p) {
   if (n == 0) return fill_u32(ctx, reinterpret_cast<uint32_t*>(n_out), 2, 0);
@@ -329,6 +332,7 @@ int select_impl(rfx_ctx* ctx, void* out, uint64_t* n_out, const void* in, uint64
     case 24: return select_vt<K, 24>(ctx, out, n_out, in, n, p);
     case 32: return select_vt<K, 32>(ctx, out, n_out, in, n, p);
   }
+  if (n <= kFewRows) return select_vt<K, 8>(ctx, out, n_out, in, n, p);
   return select_vt<K, kFVT<K>>(ctx, out, n_out, in, n, p);
 }
 

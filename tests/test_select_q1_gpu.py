@@ -54,8 +54,9 @@ def test_select_double_ops(rf, ctx, orc, op):
     assert np.array_equal(got, orc.select(rows, 8, 0, 64, op, k))
 
 
-# Tiles hold 512 x 24 rows of 8 and 16 bytes and 512 x 32 rows of narrower
-# tuples: sizes around one and two tiles, and a prime size spanning many.
+# Tiles hold 512 x 8 rows up to 65,536 rows, then 512 x 24 rows of 8 and 16
+# bytes and 512 x 32 rows of narrower tuples: sizes around whole numbers of 24
+# and 32 row tiles in small ones, and a prime size spanning many.
 @pytest.mark.parametrize("tb,n", [(8, 0), (8, 1), (8, 12287), (8, 12288), (8, 12289),
                                   (8, 24577), (8, 1_000_003), (16, 1), (16, 12287), (16, 12288),
                                   (16, 12289), (16, 24577), (16, 1_000_003), (4, 16383),
@@ -65,6 +66,19 @@ def test_select_sizes_keep_order(rf, ctx, orc, tb, n):
     shift = 8 * tb - 24  # a 16-bit field below the top byte
     got = gpu_select(rf, ctx, rows, tb, shift, 16, 3, 30_000)
     assert np.array_equal(got, orc.select(rows, tb, shift, 16, 3, 30_000))
+
+
+# The small tiles' edges, their last size and the next, and whole numbers of
+# the large tiles past it (and one row less or more).
+@pytest.mark.parametrize("n", [100, 4095, 4096, 4097, 8193, 65_535, 65_536, 65_537, 6 * 12_288, 6 * 12_288 + 1,
+                               5 * 16_384 - 1, 5 * 16_384])
+@pytest.mark.parametrize("tb", [1, 4, 8, 16])
+def test_select_tiles_by_rows(rf, ctx, orc, tb, n):
+    rows = rows_of(tb, n, 19)
+    bits = min(8 * tb, 16)
+    k = 1 << (bits - 1)
+    got = gpu_select(rf, ctx, rows, tb, 0, bits, 3, k)
+    assert np.array_equal(got, orc.select(rows, tb, 0, bits, 3, k))
 
 
 @pytest.mark.parametrize("tb", [4, 8, 16])
