@@ -84,9 +84,10 @@ __device__ __forceinline__ uint64_t wave_bound(const uint64_t* __restrict__ righ
 // where it hardly narrows anything (one block, or right keys that one round
 // tells apart).  Inside it a thread bisects: several probes a round are as many
 // comparisons one after the other (three: 300,000 x 150,000 names 136 us, 20 x
-// 10 30; one: 93 and 18).  The upper bound is the next key's lower bound,
+// 10 30; one: 93 and 16).  The upper bound is the next key's lower bound,
 // which one comparison confirms (a right key that no left key equals may lie
-// in between: then the run is galloped over).
+// in between: then the run's end is searched for).
+constexpr uint64_t kGallopFrom = 1024;
 __global__ __launch_bounds__(kSNT) void k_str_bounds(const uint64_t* __restrict__ left, uint64_t nl,
                                                      const uint64_t* __restrict__ right,
                                                      uint64_t nr, int32_t* __restrict__ lower,
@@ -116,16 +117,20 @@ __global__ __launch_bounds__(kSNT) void k_str_bounds(const uint64_t* __restrict_
   s_lo[threadIdx.x] = lo;
   __syncthreads();
   if (i >= nl) return;
-  // Every right key before `next` is not above the next left key's
-  // predecessor's range: the run of keys equal to this one ends there or
-  // before.
+  // The right keys before `next` are below the next left key (for the last
+  // one, not above the block's last), so the run of keys equal to this one ends
+  // there or before, unless the next left key is this one again (next == lo).
   const uint64_t next = i == last ? b1 : s_lo[threadIdx.x + 1];
-  uint64_t up = lo;
-  if (next > lo && !str_less(key, right[next - 1])) {
-    up = next;
-  } else {
-    // Equal keys lie in [lo, end): gallop, then search.
-    uint64_t end = b1, step = 1;
+  uint64_t up = lo, end = b1;
+  if (lo < b1) {  // one comparison for all lanes alike
+    const uint64_t at = next > lo ? next - 1 : lo;
+    const bool above = str_less(key, right[at]);
+    if (!above) up = at + 1;
+    if (above) end = at;
+    else if (next > lo) end = up;
+  }
+  if (end - up > kGallopFrom) {
+    uint64_t step = 1;
     while (up < b1) {
       const uint64_t at = up + step - 1 < b1 ? up + step - 1 : b1 - 1;
       if (str_less(key, right[at])) {
@@ -135,11 +140,11 @@ __global__ __launch_bounds__(kSNT) void k_str_bounds(const uint64_t* __restrict_
       up = at + 1;
       step <<= 1;
     }
-    while (up < end) {
-      const uint64_t mid = (up + end) >> 1;
-      if (str_less(key, right[mid])) end = mid;
-      else up = mid + 1;
-    }
+  }
+  while (up < end) {
+    const uint64_t mid = (up + end) >> 1;
+    if (str_less(key, right[mid])) end = mid;
+    else up = mid + 1;
   }
   lower[i] = static_cast<int32_t>(lo);
   count[i] = static_cast<int32_t>(up - lo);
