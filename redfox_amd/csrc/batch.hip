@@ -109,12 +109,12 @@ uint32_t grid_of(uint64_t n) {
 // Device copy: a block moves kCopyBlock bytes, all its loads in flight before
 // the first store, and runs of kCopyRun blocks are neighbours on one XCD
 // (blockIdx is dealt out to the XCDs in turn), so each XCD streams through
-// pages of its own (2 GiB 0.885 -> 0.760 ms, 1 GiB 0.418 -> 0.378; the same as
-// the runtime up to 128 MiB).
+// pages of its own (2 GiB 0.885 -> 0.760 ms, 1 GiB 0.411 -> 0.374, 256 MiB 0.100 ->
+// 0.094; 100 MiB 0.0256 and 0.0258, 65 MiB 0.0174 and 0.0181, so from 128 MiB).
 constexpr int kCopyNT = 512;
 constexpr int kCopyVT = 8;
 constexpr uint64_t kCopyBlock = 16ull * kCopyNT * kCopyVT;
-constexpr uint64_t kCopyMin = 64ull << 20;
+constexpr uint64_t kCopyMin = 128ull << 20;
 constexpr uint32_t kCopyRun = 32;
 
 __global__ __launch_bounds__(kCopyNT) void k_copy(const uint4* __restrict__ src,

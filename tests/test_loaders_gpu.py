@@ -133,7 +133,8 @@ def test_q1_plan_from_lineitem_text(rf, ctx):
         assert abs(got - want) <= 1e-12 * abs(want)
 
 
-@pytest.mark.parametrize("size", [1 << 20, (64 << 20) + 5, (64 << 20) - 16, (66 << 20) + 65_536 * 3 + 16])
+@pytest.mark.parametrize("size", [1 << 20, (64 << 20) + 5, (64 << 20) - 16, (66 << 20) + 65_536 * 3 + 16,
+                                  (128 << 20) - 16, 128 << 20, (128 << 20) + 5, (130 << 20) + 65_536 * 3 + 16])
 def test_copies_of_any_size(rf, ctx, size):
     """rfx_copy below and past the size where its own kernel takes over:
     whole blocks, a last block, last bytes, and an unaligned source."""
@@ -214,17 +215,17 @@ def test_copy_past_an_allocation_is_refused(rf, ctx, short):
     """The library's own copy kernel is not started on a range that leaves
     its allocation (the runtime's copy refused it too).  The range ends far
     beyond any memory, so the host refuses it whatever lies in between."""
-    big, small = rf.DeviceBuffer(160 << 20), rf.DeviceBuffer(70 << 20)
+    big, small = rf.DeviceBuffer(160 << 20), rf.DeviceBuffer(140 << 20)
     src, dst = (big, small) if short == "dst" else (small, big)
     with pytest.raises(rf.RfxError):
         ctx.copy(dst, src, 1 << 45)
-    ctx.copy(dst, src, 70 << 20)  # whole allocations are fine
+    ctx.copy(dst, src, 140 << 20)  # whole allocations are fine
     ctx.synchronize()
 
 
 def test_copies_within_one_buffer(rf, ctx):
     """Both ranges in one allocation, side by side up to its last byte."""
-    half = (80 << 20) + 16
+    half = (130 << 20) + 16
     buf = rf.DeviceBuffer(2 * half)
     ctx.gen_u32(buf, half // 2, 9)
     want = buf.download(np.uint8, half)
