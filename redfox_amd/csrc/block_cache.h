@@ -80,6 +80,10 @@ class BlockCache {
       auto it = blocks_.find(ptr);
       if (it == blocks_.end()) return kCallerFrees;
       if (it->second.kept) return kFreedBefore;
+      if (kept_ + it->second.size > kKeepTotal) {  // no room: no need to wait
+        blocks_.erase(it);
+        return kCallerFrees;
+      }
       // Marked before the wait below: of two threads that free it, one does.
       it->second.kept = true;
       b = it->second;
