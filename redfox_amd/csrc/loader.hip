@@ -26,9 +26,11 @@ namespace {
 
 constexpr int kLNT = 512;
 // Bytes per thread: 64 KB tiles.  Tiles take turns at one ticket word (12 ns
-// each) and at the look-back, so small tiles wait for those, large ones
-// leave the chip half empty: 133 MB of text in 16 KB tiles 118 us, 32 KB 72,
-// 64 KB 67, 128 KB 86.
+// each) and at the look-back, so small tiles wait for those; large ones take
+// longer to read where there are few.  Row ends of 133 MB of text in tiles of
+// 32 / 64 / 128 KB 67 / 50 / 42 us, of 16 MB 17 / 13 / 12, of 1.09 MB 8.2 / 9.1 / 10.8,
+// of 64 KB 8.7 / 9.0 / 10.6: 64 KB is the middle (128 KB from 16 MB on would be
+// faster still).
 constexpr int kLBytes = 128;
 constexpr int kLTile = kLNT * kLBytes;
 constexpr int kMaxFields = RFX_TBL_MAX_COLS;
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(kLNT) void k_tbl_rows(const uint8_t* __restrict__ t
 }
 
 // The newlines alone, without their places: no order, so no ticket and no
-// look-back (133 MB: 29 us against 64 by the pass above).  counts[0] is 0
+// look-back (133 MB: 29 us against 50 by the pass above).  counts[0] is 0
 // before; the last block to finish turns it into the rows.
 constexpr int kCNT = 512;
 __global__ __launch_bounds__(kCNT) void k_tbl_count(const uint8_t* __restrict__ text,
