@@ -352,7 +352,10 @@ extern "C" int rfx_select(rfx_ctx* ctx, void* out, uint64_t* n_out, const void* 
   if (op >= RFX_CMP_DLT && field_bits != 64)
     return fail(RFX_EINVAL, "rfx_select: double comparison needs a 64-bit field");
   if (n >= (1ull << 40)) return fail(RFX_ERANGE, "rfx_select: too many rows");
-  const Pred p = make_pred(field_shift, field_bits, op, constant);
+  Pred p = make_pred(field_shift, field_bits, op, constant);
+  // A shift so large that the sum above wrapped: past the tuple, where the
+  // field reads 0.
+  if (field_shift >= 128) p.shift = 0, p.mask = 0;
   switch (tuple_bytes) {
     case 1: return select_impl<uint8_t>(ctx, out, n_out, in, n, p);
     case 2: return select_impl<uint16_t>(ctx, out, n_out, in, n, p);

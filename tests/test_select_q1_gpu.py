@@ -193,3 +193,16 @@ def test_select_interval_ends(rf, ctx, orc, tb, shift, bits, op):
         got = gpu_select(rf, ctx, rows, tb, shift, bits, op, k & (2**64 - 1))
         want = orc.select(rows, tb, shift, bits, op, k & (2**64 - 1))
         assert np.array_equal(got, want), (op, hex(k))
+
+
+@pytest.mark.parametrize("tb", [1, 8, 16])
+@pytest.mark.parametrize("shift,bits", [(2**32 - 1, 2), (2**32 - 64, 64), (2**32 - 8, 8)])
+def test_select_field_past_every_tuple_reads_zero(rf, ctx, tb, shift, bits):
+    """A shift that wraps the 32-bit sum of shift and width is taken, and its
+    field has no bits of the tuple."""
+    n = 5000
+    rows = rows_of(tb, n, 60 + tb)
+    for op, k, kept in ((0, 0, n), (0, 1, 0), (1, 0, 0), (2, 1, n), (6, 1, n), (8, 0, 0), (9, 0, n)):
+        got = gpu_select(rf, ctx, rows, tb, shift, bits, op, k)
+        assert got.nbytes == kept * tb, (op, k)
+        assert kept == 0 or np.array_equal(got, rows)
