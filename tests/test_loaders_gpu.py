@@ -1,8 +1,9 @@
 """Text loading on the GPU (rfx_tbl_parse) against the oracle's parser on
 the same bytes: the reference's TC.tbl fixture, edge rows (no final
 newline, CRLF, short and empty rows, signs and spaces), texts across the
-8192-byte tile edges, an unaligned text pointer, the capacity limit, and
-the Q1 plan run from lineitem.tbl text."""
+64 KB tile edges and at every alignment, the capacity limit, and the Q1 plan
+run from lineitem.tbl text; device memory as the loader uses it: large
+copies, kept blocks, refused frees."""
 import ctypes
 import os
 
@@ -58,6 +59,13 @@ def test_tile_edge_newlines(rf, ctx):
     for L in (8190, 1, 14, 15, 16, 17, 8191, 31, 50_000, 3):  # 50000: past the LDS stage
         rows.append(b"7" * L)
     text = b"\n".join(rows) + b"\n"
+    check(rf, ctx, text, ["u32"])
+
+
+@pytest.mark.parametrize("first", [65_533, 65_534, 65_535, 65_536, 131_071])
+def test_newlines_about_tile_ends(rf, ctx, first):
+    """Empty and short rows across the end of a 64 KB tile of the row-ends pass."""
+    text = b"8" * first + b"\n\n\n12\n\n" + b"3|4\n" * 20_000
     check(rf, ctx, text, ["u32"])
 
 
