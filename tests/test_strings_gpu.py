@@ -311,7 +311,8 @@ def test_sort_strings_keys(rf, ctx, kind, rows):
                                               (700, 4097, 1, 0), (1000, 3000, 0, 1), (5, 9000, 1, 900),
                                               (256, 64, 2, 1), (300, 65, 1, 1), (300, 64, 1, 0), (1, 1, 1, 1),
                                               (257, 1, 36, 1), (255, 4000, 0, 0), (3, 1025, 0, 900),
-                                              (5, 40_000, 0, 0), (700, 1026, 0, 0), (2, 3, 100, 100)])
+                                              (5, 40_000, 0, 0), (700, 1026, 0, 0), (2, 3, 100, 100),
+                                              (5000, 10, 500, 1), (20_000, 64, 900, 1), (1025, 5000, 1, 1)])
 def test_find_bounds_string_ranges(rf, ctx, nl, nr, step, lstep):
     left = [b"key%07d" % (100 + lstep * i) for i in range(nl)]
     right = sorted(b"key%07d" % (step * (i // 3)) for i in range(nr))
