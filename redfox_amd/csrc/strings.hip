@@ -272,13 +272,17 @@ __global__ __launch_bounds__(kSNT) void k_str_stats(const uint64_t* __restrict__
     if (lane_id() == 0) atomicMax(&s_words, c);
   }
   __syncthreads();
-  // Atomics of all blocks on one word take turns (10 ns each): only a block
-  // that adds something makes them (300,000 empty strings 42 -> 30 us, 1.5 M
-  // names 194 -> 161).
+  // Atomics of all blocks on one word take turns (10 ns each): with many, only
+  // a block that adds something makes them (300,000 empty strings 42 -> 30 us,
+  // 1.5 M names 194 -> 161); with few, looking first is the longer way.
+  auto adds = [&](unsigned long long* word, unsigned long long mine, bool bits) {
+    if (!mine || gridDim.x <= kWave) return mine != 0;
+    const unsigned long long now = status_load64(reinterpret_cast<uint64_t*>(word));
+    return bits ? (mine & ~now) != 0 : mine > now;
+  };
   for (uint32_t q = threadIdx.x; q < kVaryWords; q += kSNT)
-    if (s_vary[q] & ~status_load64(reinterpret_cast<uint64_t*>(&out->vary[q])))
-      atomicOr(&out->vary[q], s_vary[q]);
-  if (threadIdx.x == 0 && s_words > status_load64(reinterpret_cast<uint64_t*>(&out->words)))
+    if (adds(&out->vary[q], s_vary[q], true)) atomicOr(&out->vary[q], s_vary[q]);
+  if (threadIdx.x == 0 && adds(&out->words, s_words, false))
     atomicMax(&out->words, static_cast<unsigned long long>(s_words));
 }
 
